@@ -18,9 +18,8 @@
 //    with allow_neg_eigval).
 //
 // Layout of the convolution: lane = 8 consecutive channels (one 16-byte bf16
-// load), wave = 512 channels, and a wave walks a run of kConvRun consecutive
-// tokens keeping the W - 1 previous inputs in registers, so each input row is
-// read once (plus W - 1 halo rows per run).  Every kernel here is HBM-bound.
+// load), wave = 512 channels of a run of 4 or 8 consecutive tokens, whose rows
+// and W - 1 halo rows it loads together.  Every kernel here is HBM-bound.
 #include "gdn_common.hpp"
 #include "gdn_kernels.h"
 
@@ -28,8 +27,12 @@ namespace kgdn {
 
 namespace {
 
-constexpr int kConvRun = 64;     // tokens per wave (a sweep of 8..256 at the model shape: 64 fastest)
 constexpr int kConvWaves = 4;
+// From this many (token, 512-channel group) rows on a wave takes eight tokens, below it four: the halo read
+// again is smaller, but fewer waves are in flight.  Measured in bf16, four against eight tokens: 18.9 / 19.6
+// us at 31,200 rows, 22.6 / 23.1 at 40,950, 29.9 / 28.9 at 65,520, 43.6 / 41.6 at 81,900, 159 / 146 at
+// 327,600; two tokens gain at most 0.4 us on the smallest inputs and lose from 10,000 rows on.
+constexpr int64_t kConvRows8 = 49152;
 
 __device__ __forceinline__ float sigmoid_f(float z) {
   return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-z * 1.4426950408889634f));
@@ -67,105 +70,109 @@ __device__ __forceinline__ void seq_of(int64_t t, const ConvArgs& a, int& n, int
   eos = a.cu[lo + 1];
 }
 
-template <typename TX, int W, int HL>
-__global__ __launch_bounds__(WAVE * kConvWaves) void conv1d_kernel(ConvArgs a, int64_t n_runs) {
-  const int64_t wv = (int64_t)blockIdx.x * kConvWaves + threadIdx.x / WAVE;
+// A wave takes R consecutive tokens of 512 channels.  Bound by HBM on large inputs and by the latency of
+// one wave on small ones, so a wave sends all its R + W - 1 row loads at once: walking a run of 64 rows
+// with the window in registers, each row waited for in turn, took 52 us at T = 1560, D = 5120 (now 12.5)
+// and 304 us at T = 32760, D = 10240 (now 277 us = 4.8 TB/s; a plain copy reaches 5.1).  The halo rows are
+// read again by the next wave, the workgroup's next, from the caches.
+template <typename TX, int W, int HL, int R>
+__global__ __launch_bounds__(WAVE * kConvWaves) void conv1d_rows_kernel(ConvArgs a, int64_t n_runs, int fold_state) {
+  // the workgroup's waves take consecutive runs of one channel group, which share their halo rows
   const int ncg = (a.D + 511) / 512;
-  const int64_t run = wv / ncg;
+  const int64_t run = (int64_t)(blockIdx.x / ncg) * kConvWaves + threadIdx.x / WAVE;
   if (run >= n_runs) return;
-  const int l = lane_id();
-  const int c0 = (int)(wv % ncg) * 512 + 8 * l;
+  const int c0 = (int)(blockIdx.x % ncg) * 512 + 8 * lane_id();
   const bool ok = c0 < a.D;
-  const int64_t t_begin = run * kConvRun;
-  const int64_t t_stop = min(t_begin + (int64_t)kConvRun, a.total_tokens);
+  const int cc = ok ? c0 : 0;                        // lanes past D load channel 0 and store nothing
+  const int64_t t_begin = run * R;
+  const int64_t t_stop = min(t_begin + (int64_t)R, a.total_tokens);
   const TX* x = static_cast<const TX*>(a.x);
   TX* y = static_cast<TX*>(a.y);
-
-  // taps of the lane's 8 channels: 8 W consecutive elements of weight [D, W], read 8 at a time
+  constexpr int P = W - 1;
+  // rows t_begin - P .. t_begin + R - 1, clamped into the tensor (a clamped row reaches no output)
+  Vec8<TX> row[R + P];
+#pragma unroll
+  for (int i = 0; i < R + P; ++i) {
+    const int64_t s = t_begin - P + i;
+    row[i] = ld8<TX>(x + (s < 0 ? 0 : s < t_stop ? s : t_stop - 1) * a.D + cc);
+  }
   float wt[W][8], bias[8];
 #pragma unroll
   for (int q = 0; q < W; ++q) {
-    float w8[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (ok) {
-      if (a.w_dtype == DT_F32) ld_row8<float>(static_cast<const float*>(a.w) + (int64_t)c0 * W + 8 * q, w8);
-      else ld_row8<bf16>(static_cast<const bf16*>(a.w) + (int64_t)c0 * W + 8 * q, w8);
-    }
+    float w8[8];
+    if (a.w_dtype == DT_F32) ld_row8<float>(static_cast<const float*>(a.w) + (int64_t)cc * W + 8 * q, w8);
+    else ld_row8<bf16>(static_cast<const bf16*>(a.w) + (int64_t)cc * W + 8 * q, w8);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int f = 8 * q + e;                       // flat index (channel c0 + f / W, tap f % W)
-      wt[f % W][f / W] = w8[e];
-    }
+    for (int e = 0; e < 8; ++e) wt[(8 * q + e) % W][(8 * q + e) / W] = w8[e];
   }
 #pragma unroll
   for (int e = 0; e < 8; ++e) bias[e] = 0.f;
-  if (a.bias && ok) ld_chan8(a.bias, c0, a.w_dtype, bias);
+  if (a.bias) ld_chan8(a.bias, cc, a.w_dtype, bias);
 
   int n;
   int64_t bos, eos;
   seq_of(t_begin, a, n, bos, eos);
-  // window: win[i] = x~[t - (W - 1) + i], i < W - 1
-  float win[W > 1 ? W - 1 : 1][8];
-  auto fill_window = [&](int64_t t) {
+  // the cache of sequence n, read where a window starts before the sequence: all loads in one batch
+  float hc[8 * W];
+  auto load_cache = [&]() {
 #pragma unroll
-    for (int i = 0; i < W - 1; ++i) {
-      const int64_t s = t - (W - 1) + i;
+    for (int f = 0; f < 8 * W; ++f) hc[f] = 0.f;
+    if (a.h0) {
+      const TX* h = static_cast<const TX*>(a.h0) + ((int64_t)n * a.D + cc) * W;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) win[i][e] = 0.f;
-      if (!ok) continue;
-      if (s >= bos) {
-        ld_row8<TX>(x + s * a.D + c0, win[i]);
-      } else if (a.h0 && s - bos + W >= 0) {       // cache slot of x~[s]
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          win[i][e] = ld_scalar(a.h0, ((int64_t)n * a.D + c0 + e) * W + (s - bos + W), a.x_dtype);
-      }
+      for (int f = 0; f < 8 * W; ++f) hc[f] = to_f32(h[f]);
     }
   };
-  fill_window(t_begin);
-
-  for (int64_t t = t_begin; t < t_stop; ++t) {
-    if (t >= eos) {                                 // next sequence (varlen): restart the window
-      seq_of(t, a, n, bos, eos);
-      fill_window(t);
-    }
-    float cur[8];
+  if (t_begin - P < bos) load_cache();
 #pragma unroll
-    for (int e = 0; e < 8; ++e) cur[e] = 0.f;
-    if (ok) ld_row8<TX>(x + t * a.D + c0, cur);
+  for (int r = 0; r < R; ++r) {
+    const int64_t t = t_begin + r;
+    if (t >= t_stop) break;
+    if (t >= eos) {
+      seq_of(t, a, n, bos, eos);
+      load_cache();
+    }
+    float in[W][8];                                  // x~[t - P + i]
+#pragma unroll
+    for (int i = 0; i < W; ++i)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) in[i][e] = vget<TX>(row[r + i], e);
+#pragma unroll
+    for (int d = 0; d < P; ++d)                      // the sequence's d-th token: P - d inputs from the cache
+      if (t - bos == d) {
+#pragma unroll
+        for (int i = 0; i < P - d; ++i)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) in[i][e] = hc[e * W + d + 1 + i];
+      }
     float out[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       float acc = bias[e];
 #pragma unroll
-      for (int i = 0; i < W - 1; ++i) acc = fmaf(wt[i][e], win[i][e], acc);
-      acc = fmaf(wt[W - 1][e], cur[e], acc);
+      for (int i = 0; i < W; ++i) acc = fmaf(wt[i][e], in[i][e], acc);
       if (a.silu) acc = acc * sigmoid_f(acc);
       out[e] = round_to<TX>(acc);
     }
-    if constexpr (HL > 0) {                         // per-head L2 norm over HL lanes of 8 channels
+    if constexpr (HL > 0) {                          // per-head L2 norm over HL lanes of 8 channels
       float ss = 0.f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) ss = fmaf(out[e], out[e], ss);
 #pragma unroll
       for (int off = HL / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off, HL);
-      const float r = 1.0f / __builtin_sqrtf(ss + 1e-6f);
+      const float r1 = 1.0f / __builtin_sqrtf(ss + 1e-6f);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) out[e] *= r;
+      for (int e = 0; e < 8; ++e) out[e] *= r1;
     }
-    if (ok) {
-      Vec8<TX> o;
+    if (!ok) continue;
+    Vec8<TX> o;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) vset<TX>(o, e, out[e]);
-      st8<TX>(y + t * a.D + c0, o);
-    }
+    for (int e = 0; e < 8; ++e) vset<TX>(o, e, out[e]);
+    st8<TX>(y + t * a.D + c0, o);
+    if (fold_state && t == eos - 1) {                // the final cache: the last token's own window
+      TX* ht = static_cast<TX*>(a.ht) + ((int64_t)n * a.D + c0) * W;
 #pragma unroll
-    for (int i = 0; i + 1 < W - 1; ++i) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) win[i][e] = win[i + 1][e];
-    }
-    if constexpr (W > 1) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) win[W - 2][e] = cur[e];
+      for (int f = 0; f < 8 * W; ++f) ht[f] = from_f32<TX>(in[f % W][f / W]);
     }
   }
 }
@@ -214,13 +221,16 @@ __global__ __launch_bounds__(256) void to_f32_kernel(const void* src, int dt, fl
   if (i < n) dst[i] = ld_scalar(src, i, dt);
 }
 
-template <typename TX, int W>
-int launch_conv_w(const ConvArgs& a, int64_t n_runs, hipStream_t s) {
-  const int64_t waves = n_runs * ((a.D + 511) / 512);
-  const dim3 grid((unsigned)((waves + kConvWaves - 1) / kConvWaves));
+template <typename TX, int W, int R>
+int launch_conv_rows(const ConvArgs& a, bool fold, hipStream_t s) {
+  const int64_t n_runs = (a.total_tokens + R - 1) / R;
+  const int64_t blocks = (n_runs + kConvWaves - 1) / kConvWaves * ((a.D + 511) / 512);
   switch (a.head_lanes) {
-#define KGDN_CONV_CASE(HL) \
-    case HL: hipLaunchKernelGGL((conv1d_kernel<TX, W, HL>), grid, dim3(WAVE * kConvWaves), 0, s, a, n_runs); break;
+#define KGDN_CONV_CASE(HL)                                                                                     \
+    case HL:                                                                                                   \
+      hipLaunchKernelGGL((conv1d_rows_kernel<TX, W, HL, R>), dim3((unsigned)blocks), dim3(WAVE * kConvWaves),  \
+                         0, s, a, n_runs, (int)fold);                                                          \
+      break;
     KGDN_CONV_CASE(0) KGDN_CONV_CASE(8) KGDN_CONV_CASE(16) KGDN_CONV_CASE(32) KGDN_CONV_CASE(64)
 #undef KGDN_CONV_CASE
     default: return -2;
@@ -230,24 +240,22 @@ int launch_conv_w(const ConvArgs& a, int64_t n_runs, hipStream_t s) {
 
 template <typename TX>
 int launch_conv_t(const ConvArgs& a, hipStream_t s) {
-  const int64_t n_runs = (a.total_tokens + kConvRun - 1) / kConvRun;
-  if (n_runs > 0) {
+  // fixed-length sequences: the wave of a sequence's last token writes its final cache; a varlen batch may
+  // hold empty sequences, which no wave visits
+  const bool fold = a.ht != nullptr && a.cu == nullptr && a.total_tokens > 0;
+  if (a.total_tokens > 0) {
+    const bool r8 = a.total_tokens * ((a.D + 511) / 512) >= kConvRows8;
     int rc = -2;
     switch (a.W) {
-      case 1: rc = launch_conv_w<TX, 1>(a, n_runs, s); break;
-      case 2: rc = launch_conv_w<TX, 2>(a, n_runs, s); break;
-      case 3: rc = launch_conv_w<TX, 3>(a, n_runs, s); break;
-      case 4: rc = launch_conv_w<TX, 4>(a, n_runs, s); break;
+      case 1: rc = launch_conv_rows<TX, 1, 4>(a, fold, s); break;
+      case 2: rc = launch_conv_rows<TX, 2, 4>(a, fold, s); break;
+      case 3: rc = launch_conv_rows<TX, 3, 4>(a, fold, s); break;
+      case 4: rc = r8 ? launch_conv_rows<TX, 4, 8>(a, fold, s) : launch_conv_rows<TX, 4, 4>(a, fold, s); break;
       default: return -2;
     }
-    if (rc) return rc;
+    if (rc || fold) return rc;
   }
-  if (a.ht && a.N > 0) {
-    const int64_t total = (int64_t)a.N * a.D;
-    hipLaunchKernelGGL(conv_state_kernel<TX>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, a);
-    if (hipGetLastError() != hipSuccess) return -1;
-  }
-  return 0;
+  return launch_conv_state(a, s);
 }
 
 }  // namespace

@@ -150,6 +150,23 @@ def test_gpu_causal_conv1d(cid, B, T, D, W, cu, cache, dt, l2):
     np.testing.assert_array_equal(hf.float().cpu().numpy(), h_r)
 
 
+# Runs of 4 and (from 49152 rows of 512 channels) 8 tokens: sequences shorter than, equal to and one past a
+# run, sequences ending or starting inside one, and a short last run.
+CONV_RUN_CASES = [
+    ("batch_t1", 5, 1, 72, 4, None, "bf16"), ("batch_t3", 3, 3, 520, 4, None, "fp32"),
+    ("batch_t4", 3, 4, 512, 4, None, "bf16"), ("batch_t5", 7, 5, 1032, 4, None, "bf16"),
+    ("w1", 2, 6, 72, 1, None, "bf16"), ("w2", 2, 7, 72, 2, None, "fp32"),
+    ("varlen", 1, 21, 520, 4, [0, 1, 1, 4, 8, 9, 21], "bf16"),
+    ("runs8", 3, 820, 10240, 4, None, "bf16"), ("runs8_varlen", 1, 2461, 10240, 4, [0, 2, 1207, 2461], "bf16"),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cid,B,T,D,W,cu,dt", CONV_RUN_CASES, ids=[c[0] for c in CONV_RUN_CASES])
+def test_gpu_conv_run_edges(cid, B, T, D, W, cu, dt):
+    test_gpu_causal_conv1d(cid, B, T, D, W, cu, True, dt, 0)
+
+
 @pytest.mark.gpu
 def test_gpu_short_convolution_module_prefill_then_decode():
     import kairos_gdn
