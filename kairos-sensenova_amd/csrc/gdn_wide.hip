@@ -987,7 +987,8 @@ __global__ __launch_bounds__(NT_F + FL * WAVE) void wide_dhu_kernel(BwdArgs a, i
     wait_all_loads();
     // vmcnt counts in issue order; the waits below name how many of this wave's operations issued after
     // the ones waited for may still be in flight: the q^T / do loads (10), the prefetch (1, loader 3: 2),
-    // the dv2 stores (2), the w^T / dv_local loads (10), the snapshot stores (8).  The snapshot leaves
+    // the dv2 stores (2; a wave with no row inside a short chunk skips them, so after the ragged last chunk
+    // they are not counted), the w^T / dv_local loads (10), the snapshot stores (8).  The snapshot leaves
     // after B1h, a half step before the next chunk's k loads: issued beside them (after B2) its stores
     // held those loads back by about the length of the second half (measured).
     static_assert(32 / FL == 8 && 8 / FL == 2, "the wait counts below assume four loader waves");
@@ -997,12 +998,8 @@ __global__ __launch_bounds__(NT_F + FL * WAVE) void wide_dhu_kernel(BwdArgs a, i
       if (it < top) {
         store_dv(it + 1);                                 // the stores first, then this half's loads
         load_b(it);
-        if (it >= 1) {                                    // the previous step prefetched chunk it - 1
-          if (lw == 3) wait_loads_but<2 + 2 + 10>();
-          else wait_loads_but<1 + 2 + 10>();
-        } else {
-          wait_loads_but<2 + 10>();
-        }
+        const int pf = it >= 1 ? (lw == 3 ? 2 : 1) : 0;   // the previous step prefetched chunk it - 1
+        wait_loads_but_n(pf + (chunk_nv(it + 1) == C ? 2 : 0) + 10);
       } else {
         load_b(it);
         wait_loads_but<10>();                             // the prologue's loads are complete

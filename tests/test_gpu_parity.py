@@ -648,3 +648,33 @@ def test_streaming_fp8_rollout():
     drift = rel(host(state)[:, dheads], h_single)
     note(f"    end-state drift vs single-call fp32 (unquantised q/k): {drift:.3e}")
     assert math.isfinite(drift) and drift < 0.05
+
+
+@pytest.mark.parametrize("lens", [[70], [64, 64, 1], [0, 130, 0, 65, 128, 63], [1 + 67 * (i % 3) for i in range(64)],
+                                  [(37 * i) % 131 for i in range(65)]], ids=["n1", "ties", "empty", "n64", "n65"])
+@pytest.mark.parametrize("H,V", [(1, 64), (3, 192)])
+def test_wide_varlen_order(lens, H, V):
+    """K = 256 packed sequences are walked longest first (up to 64 of them), each head's value tiles over the
+    XCDs: every sequence's o, final state and gradients have the bits of a call of its own."""
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    x = make_inputs(1, int(cu[-1]), H, 256, V, seed=len(lens) + V, n_states=len(lens))
+    t = to_dev(x, "bf16")
+    gen = torch.Generator().manual_seed(1)
+    do = torch.randn(t["v"].shape, generator=gen).cuda().to(torch.bfloat16)
+    dht = torch.randn(t["h0"].shape, generator=gen).cuda()
+
+    def both(q, k, v, g, beta, h0, do, dht, cu):
+        y = [a.detach().clone().requires_grad_() for a in (q, k, v, g, beta, h0)]
+        o, ht = kairos_gdn.chunk_gated_delta_rule(*y[:5], initial_state=y[5], output_final_state=True, cu_seqlens=cu)
+        return [o, ht, *torch.autograd.grad([o, ht], y, [do, dht])]
+
+    names = ("q", "k", "v", "g", "beta")
+    got = both(*(t[a] for a in names), t["h0"], do, dht, torch.from_numpy(cu).cuda())
+    note(f"varlen order: {len(lens)} sequences H={H} V={V}")
+    for n, (b, e) in enumerate(zip(cu[:-1], cu[1:])):
+        if e == b:
+            assert torch.equal(got[1][n], t["h0"][n])
+            continue
+        one = both(*(t[a][:, b:e] for a in names), t["h0"][n:n + 1], do[:, b:e], dht[n:n + 1], None)
+        for i, (a, w) in enumerate(zip(got, one)):
+            assert torch.equal(a[n:n + 1] if i in (1, 7) else a[:, b:e], w), (n, b, e, i)
