@@ -224,6 +224,35 @@ __device__ __forceinline__ void ld_tile64(const unsigned char* base, uint32_t ro
   dma16_(base, rr * row_bytes + 16u * (pos ^ (kSwzA ? swz_a(r) : swz_v(r))), dst + 1024u * i);
 }
 
+// ---------------------------------------------------------------------------
+// which (sequence, head, value tile) a workgroup takes
+// ---------------------------------------------------------------------------
+// Workgroup b runs on XCD b % 8 and workgroups start in order of b.  The H V / 64 units of one sequence
+// are spread over the XCDs in runs, so that the value tiles of a head share an XCD's L2 (q, w, k^T, Aqk,
+// Ai) while every XCD takes part in every sequence; sequences follow each other, in a varlen batch of at
+// most 64 the longest first, since the last one to start decides when the kernel ends.  A packed batch of
+// 24, 1, 49 and 99 chunks with 20 heads: 786 us with whole sequences laid over the XCDs (the longest held
+// by two of them, three rounds of its 99 chunks), 426 us so.
+__device__ __forceinline__ bool wide_unit(const int64_t* cu, int N, int units, int& n, int& idx) {
+  const int per_xcd = (units + 7) / 8;
+  const int j = blockIdx.x / 8;
+  idx = (blockIdx.x % 8) * per_xcd + j % per_xcd;
+  n = j / per_xcd;
+  if (idx >= units) return false;
+  if (cu != nullptr && N > 1 && N <= WAVE) {              // the sequence of rank n by length, one per lane
+    const int l = lane_id(), lm = min(l, N - 1);
+    const int64_t len = cu[lm + 1] - cu[lm];
+    const int chunks = (int)((len + C - 1) / C);
+    int rank = 0;
+    for (int i = 0; i < N; ++i) {
+      const int ci = __builtin_amdgcn_readlane(chunks, i);
+      rank += ci > chunks || (ci == chunks && i < l) ? 1 : 0;
+    }
+    n = __builtin_ctzll(__ballot(l < N && rank == n));
+  }
+  return true;
+}
+
 // kRc: the backward's recompute of the forward (chunk_delta_h.py:52-224 alone): the state before each
 // chunk (bf16, through the q half of the w / q tile, which q does not use here) and v_new (through the o
 // tile) leave as whole rows stored by the loader waves; q, Aqk and the output products are skipped.
@@ -233,7 +262,7 @@ __device__ __forceinline__ void ld_tile64(const unsigned char* base, uint32_t ro
 constexpr int kNormSpinMax = 1 << 14;
 
 template <bool kRc, bool kNorm>
-__global__ __launch_bounds__(NT_F + FL * WAVE) void wide_fused_kernel(WideFusedArgs a, int V, int total_units) {
+__global__ __launch_bounds__(NT_F + FL * WAVE) void wide_fused_kernel(WideFusedArgs a, int V) {
   // LDS: w and q of the chunk (adjacent: q reads are w reads + 32 KB), k^T of the chunk, and two
   // buffer sets of the chunk's small tiles: Aqk, Ai, the v tile of the workgroup's 64 columns, gc, beta
   __shared__ __align__(16) bf16 s_wq[2 * C * FK];
@@ -248,16 +277,12 @@ __global__ __launch_bounds__(NT_F + FL * WAVE) void wide_fused_kernel(WideFusedA
   __shared__ __align__(16) float s_pf[WAVE];              // landing words of the L2 prefetch
   constexpr uint32_t QOFF = C * FK * 2, ABUF = C * C * 2, GBUF = C * 4;
 
-  // XCD-aware order: the V tiles of one head run on one XCD and share its q, w, k^T, Aqk, Ai in L2
-  const int per_xcd = gridDim.x / 8;
-  const int o_idx = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-  if (o_idx >= total_units) return;
-  const int nvt = V / FVT;
-  const int unit = o_idx / nvt;
-  const int H = a.H;
-  const int n = unit / H, h = unit % H;
+  const int nvt = V / FVT, H = a.H;
+  int n, idx;
+  if (!wide_unit(a.cu, a.N, H * nvt, n, idx)) return;
+  const int h = idx / nvt;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), l = lane_id(), lg = l >> 4, lc = l & 15;
-  const int vt0 = __builtin_amdgcn_readfirstlane((o_idx % nvt) * FVT);    // the workgroup's first column
+  const int vt0 = __builtin_amdgcn_readfirstlane((idx % nvt) * FVT);      // the workgroup's first column
 
   int64_t bos, eos, c_first;
   if (a.cu == nullptr) {
@@ -870,20 +895,17 @@ constexpr uint32_t PF_OFF = G_OFF + 2 * C * 4;       // landing words of the L2 
 constexpr uint32_t TOTAL = PF_OFF + WAVE * 4;
 }  // namespace dhu_lds
 
-__global__ __launch_bounds__(NT_F + FL * WAVE) void wide_dhu_kernel(BwdArgs a, int V, int total_units) {
+__global__ __launch_bounds__(NT_F + FL * WAVE) void wide_dhu_kernel(BwdArgs a, int V) {
   using namespace dhu_lds;
   __shared__ __align__(16) unsigned char smem[TOTAL];
   const uint32_t base = lds_u32(smem);
 
-  const int per_xcd = gridDim.x / 8;                      // XCD-aware order, as the forward
-  const int o_idx = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-  if (o_idx >= total_units) return;
-  const int nvt = V / FVT;
-  const int unit = o_idx / nvt;
-  const int H = a.H;
-  const int n = unit / H, h = unit % H;
+  const int nvt = V / FVT, H = a.H;
+  int n, idx;
+  if (!wide_unit(a.cu, a.N, H * nvt, n, idx)) return;
+  const int h = idx / nvt;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), l = lane_id(), lg = l >> 4, lc = l & 15;
-  const int vt0 = __builtin_amdgcn_readfirstlane((o_idx % nvt) * FVT);
+  const int vt0 = __builtin_amdgcn_readfirstlane((idx % nvt) * FVT);
 
   int64_t bos, eos, c_first;
   if (a.cu == nullptr) {
@@ -1599,10 +1621,9 @@ bool wide_dhu_supported(int compute_dtype, int K, int V) {
 
 int launch_wide_dhu(const BwdArgs& a, int V, hipStream_t s) {
   if (V % FVT != 0 || !a.qT || !a.wT || !a.dh || !a.dv2) return -2;
-  const int total = a.N * a.H * (V / FVT);
-  if (total == 0) return 0;
-  const int grid = (total + 7) / 8 * 8;
-  hipLaunchKernelGGL(wide_dhu_kernel, dim3(grid), dim3(NT_F + FL * WAVE), 0, s, a, V, total);
+  if (a.N * a.H == 0) return 0;
+  const int grid = a.N * ((a.H * (V / FVT) + 7) / 8 * 8);   // wide_unit
+  hipLaunchKernelGGL(wide_dhu_kernel, dim3(grid), dim3(NT_F + FL * WAVE), 0, s, a, V);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -1622,16 +1643,15 @@ int launch_wide_dqkwg(const BwdArgs& a, int K, int V, int64_t nc_grid, hipStream
 
 int launch_wide_fused(const WideFusedArgs& a, int V, hipStream_t s) {
   if (V % FVT != 0 || a.N * a.H == 0) return -2;
-  const int total = a.N * a.H * (V / FVT);
-  const int grid = (total + 7) / 8 * 8;
+  const int grid = a.N * ((a.H * (V / FVT) + 7) / 8 * 8);   // wide_unit
   if (a.h_out) {
     if (!a.vn_out || a.ht || a.ngate) return -2;
-    hipLaunchKernelGGL((wide_fused_kernel<true, false>), dim3(grid), dim3(NT_F + FL * WAVE), 0, s, a, V, total);
+    hipLaunchKernelGGL((wide_fused_kernel<true, false>), dim3(grid), dim3(NT_F + FL * WAVE), 0, s, a, V);
   } else if (a.ngate) {
     if (V > 8 * FVT || a.nss == nullptr) return -2;
-    hipLaunchKernelGGL((wide_fused_kernel<false, true>), dim3(grid), dim3(NT_F + FL * WAVE), 0, s, a, V, total);
+    hipLaunchKernelGGL((wide_fused_kernel<false, true>), dim3(grid), dim3(NT_F + FL * WAVE), 0, s, a, V);
   } else {
-    hipLaunchKernelGGL((wide_fused_kernel<false, false>), dim3(grid), dim3(NT_F + FL * WAVE), 0, s, a, V, total);
+    hipLaunchKernelGGL((wide_fused_kernel<false, false>), dim3(grid), dim3(NT_F + FL * WAVE), 0, s, a, V);
   }
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
