@@ -335,34 +335,37 @@ size_t bwd_ws(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t n_s
 // reference's stage order with its intermediates in the workspace.  Used for the
 // shapes the fused kernels do not cover: fp32, and the Kairos model's head dims
 // K = 256, V = 512 (any K in {64, 128, 256} with V a multiple of 16).
-// The pipelined form of the fused K = 256 path: the chunks of every sequence are cut into P parts
-// (4 by default, growing by 1.4 along the sequence);
-// the prepare kernel of part p + 1 runs on a second stream while the recurrence walks part p (whose
-// 64-column workgroups leave CUs idle: 160 of 256 at the Kairos layer shape), the state passing
-// between parts through an fp32 buffer.  KAIROS_GDN_WIDE_PIPE sets P (1: one prepare, then one
-// recurrence); fixed-length sequences only.  Part 0's prepare runs on the caller's stream (the whole
-// GPU), the later prepares on a second stream and the recurrence parts on a third.  Prepare p + 1
-// waits for an event recorded just before recurrence part p (wide_mark_mode), so the recurrence's
-// workgroups are dispatched first and the prepare fills the CUs they leave (were both ready at once,
-// the prepare's 10^4 workgroups could take every CU and hold the recurrence back).  The caller's
-// stream waits for the last recurrence part.
+// The pipelined form of the fused K = 256 path: the chunks of every sequence are cut into P parts, growing
+// along the sequence; the prepare kernel of part p + 1 runs on a second stream while the recurrence walks
+// part p on the caller's stream (its 64-column workgroups leave CUs idle: 160 of 256 taken at the Kairos layer
+// shape), the state passing between parts through an fp32 buffer.  Fixed-length sequences only.  Prepare
+// p + 1 waits for an event recorded just before recurrence part p (wide_mark_mode), so the recurrence's
+// workgroups are dispatched first and the prepare fills the CUs they leave (were both ready at once, the
+// prepare's 10^4 workgroups could take every CU and hold the recurrence back).
 constexpr int kMaxParts = 16;
 
-int wide_pipe_parts() {
-  const char* e = std::getenv("KAIROS_GDN_WIDE_PIPE");
-  if (e == nullptr) return 4;
-  const int p = std::atoi(e);
-  return p < 1 ? 1 : p > kMaxParts ? kMaxParts : p;
-}
-
-// Part sizes grow by this factor (KAIROS_GDN_WIDE_PIPE_GROWTH; 1 = equal parts): part 0's prepare
-// runs alone, so a smaller first part shortens the call as long as each later part's prepare, on
-// the CUs the recurrence leaves, still finishes within the previous recurrence part.
-double wide_pipe_growth() {
-  const char* e = std::getenv("KAIROS_GDN_WIDE_PIPE_GROWTH");
-  if (e == nullptr) return 1.4;
-  const double g = std::atof(e);
-  return g < 0.25 ? 0.25 : g > 4.0 ? 4.0 : g;
+// Parts and their growth.  A part boundary costs the caller's stream about 16 us of waits, and what it hides
+// is the prepare of the later parts (about 0.05 us per (chunk, head) on all CUs), so short calls run in one
+// part: with 20 heads 188 -> 99 us at 25 chunks and 294 -> 225 us at 64 against four parts, one and two parts
+// equal (434 us) at 128, two ahead at 256 (795 against 849, three 793, four 808) and four at 512 (1499, two
+// 1543, one 1667).  Where the recurrence takes at most half of the CUs the later prepares run on the others
+// several times faster than it walks, so the first part can be small: two parts growing by 3, from 1280
+// items on (10 heads, 128 chunks: 372 against 379 us; 512 chunks: 1353, four parts by 1.4 1371, one 1443; 5
+// heads, 512 chunks: 1306, 1343, 1347).  KAIROS_GDN_WIDE_PIPE sets P, KAIROS_GDN_WIDE_PIPE_GROWTH the growth.
+void wide_pipe_plan(int64_t nt, int64_t seq_heads, int64_t vtiles, int* parts, double* growth) {
+  const int64_t items = nt * seq_heads;
+  const bool half_free = 2 * seq_heads * vtiles <= device_cus();
+  *growth = half_free ? 3.0 : 1.4;
+  *parts = half_free ? (items >= 1280 ? 2 : 1) : items >= 8192 ? 4 : items >= 3072 ? 2 : 1;
+  if (const char* e = std::getenv("KAIROS_GDN_WIDE_PIPE")) {
+    const int p = std::atoi(e);
+    *parts = p < 1 ? 1 : p > kMaxParts ? kMaxParts : p;
+    *growth = 1.4;
+  }
+  if (const char* e = std::getenv("KAIROS_GDN_WIDE_PIPE_GROWTH")) {
+    const double g = std::atof(e);
+    *growth = g < 0.25 ? 0.25 : g > 4.0 ? 4.0 : g;
+  }
 }
 
 // Chunk boundaries of P parts of nt chunks with sizes growing by `growth`: b[0] = 0, b[P] = nt, every
@@ -382,7 +385,7 @@ void wide_pipe_bounds(int64_t nt, int P, double growth, int64_t* b) {
 }
 
 std::mutex g_aux_mu;                                     // held while a pipelined call enqueues its work
-hipStream_t g_aux_stream[64][4] = {};
+hipStream_t g_aux_stream[64][3] = {};
 hipEvent_t g_aux_events[64][3 * kMaxParts + 4] = {};   // + 4 join events
 
 // What releases prepare p + 1 (KAIROS_GDN_WIDE_PIPE_MARK): 0, a one-workgroup marker kernel on the
@@ -400,7 +403,7 @@ int wide_mark_mode() {
 // The four streams (prepares, recurrence parts, markers, the per-part gated norm) and the events of
 // the current device, created on first use and kept until the process ends (a recorded event may be
 // recorded again: waits already enqueued keep the record they saw).  Call with g_aux_mu held.
-int aux_streams(hipStream_t* sp, hipStream_t* sr, hipStream_t* sm, hipStream_t* sn, hipEvent_t** events) {
+int aux_streams(hipStream_t* sp, hipStream_t* sm, hipStream_t* sn, hipEvent_t** events) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return -1;
   if (g_aux_events[dev][0] == nullptr) {
@@ -409,15 +412,14 @@ int aux_streams(hipStream_t* sp, hipStream_t* sr, hipStream_t* sm, hipStream_t* 
   }
   *events = g_aux_events[dev];
   if (g_aux_stream[dev][0] == nullptr) {
-    hipStream_t st[4] = {nullptr, nullptr, nullptr, nullptr};
-    for (int j = 0; j < 4; ++j)
+    hipStream_t st[3] = {nullptr, nullptr, nullptr};
+    for (int j = 0; j < 3; ++j)
       if (hipStreamCreateWithFlags(&st[j], hipStreamNonBlocking) != hipSuccess) return -1;
-    for (int j = 0; j < 4; ++j) g_aux_stream[dev][j] = st[j];
+    for (int j = 0; j < 3; ++j) g_aux_stream[dev][j] = st[j];
   }
   *sp = g_aux_stream[dev][0];
-  *sr = g_aux_stream[dev][1];
-  *sm = g_aux_stream[dev][2];
-  *sn = g_aux_stream[dev][3];
+  *sm = g_aux_stream[dev][1];
+  *sn = g_aux_stream[dev][2];
   return 0;
 }
 
@@ -528,22 +530,23 @@ int run_staged(const Geometry& G, const void* q, const void* k, const void* v, c
   }
   if (wide && G.nc > 0 && may_fork && cu_seqlens == nullptr) {
     const int64_t nt = (G.T + kgdn::C - 1) / kgdn::C;
-    int P = wide_pipe_parts();
+    int P = 1;
+    double growth = 1.0;
+    wide_pipe_plan(nt, (int64_t)N * H, V / 64, &P, &growth);
     if (nt < 2 * P) P = 1;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (P > 1 && (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)) P = 1;
     std::unique_lock<std::mutex> lk(g_aux_mu, std::defer_lock);
-    hipStream_t s2 = nullptr, s3 = nullptr, s4 = nullptr, s5 = nullptr;
+    hipStream_t s2 = nullptr, s4 = nullptr, s5 = nullptr;
     hipEvent_t* ev = nullptr;
     if (P > 1) {
       lk.lock();
-      if (aux_streams(&s2, &s3, &s4, &s5, &ev) != 0) {
+      if (aux_streams(&s2, &s4, &s5, &ev) != 0) {
         lk.unlock();
         P = 1;
       }
     }
     if (P > 1) {
-      const double growth = wide_pipe_growth();
       int64_t bnd[kMaxParts + 1];
       if (growth == 1.0) {
         const int64_t span = (nt + P - 1) / P;
@@ -580,7 +583,7 @@ int run_staged(const Geometry& G, const void* q, const void* k, const void* v, c
       };
       prepare(0, s);
       for (int p = 0; p < P && rc == KAIROS_GDN_OK; ++p) {
-        wait(s3, ev[p]);
+        if (p > 0) wait(s, ev[p]);
         if (p + 1 < P) {
           if (beside) {                                   // the marker waits for what part p waits for
             wait(s4, ev[p]);
@@ -588,8 +591,8 @@ int run_staged(const Geometry& G, const void* q, const void* k, const void* v, c
             if (rc == KAIROS_GDN_OK) rc = from_launch(kgdn::launch_marker(s4), "marker");
             record(ev[kMaxParts + p], s4);
           } else {
-            if (mark == 0 && rc == KAIROS_GDN_OK) rc = from_launch(kgdn::launch_marker(s3), "marker");
-            record(ev[kMaxParts + p], s3);
+            if (mark == 0 && rc == KAIROS_GDN_OK) rc = from_launch(kgdn::launch_marker(s), "marker");
+            record(ev[kMaxParts + p], s);
           }
         }
         kgdn::WideFusedArgs fp = fa;
@@ -600,8 +603,8 @@ int run_staged(const Geometry& G, const void* q, const void* k, const void* v, c
           fp.h0_dtype = KAIROS_GDN_F32;
         }
         if (p + 1 < P) fp.ht = st;
-        if (rc == KAIROS_GDN_OK) rc = from_launch(kgdn::launch_wide_fused(fp, V, s3), "wide fused recurrence");
-        if ((beside && p + 2 < P) || nparts) record(ev[2 * kMaxParts + p], s3);
+        if (rc == KAIROS_GDN_OK) rc = from_launch(kgdn::launch_wide_fused(fp, V, s), "wide fused recurrence");
+        if ((beside && p + 2 < P) || nparts) record(ev[2 * kMaxParts + p], s);
         if (p + 1 < P) {
           wait(s2, ev[kMaxParts + p]);
           prepare(p + 1, s2);
@@ -614,20 +617,21 @@ int run_staged(const Geometry& G, const void* q, const void* k, const void* v, c
         norm_part(P - 1);
       }
       // Join, also after a failed launch or event call above: the caller's stream waits for all
-      // that was queued on the library streams (prepares on s2, recurrence parts on s3, markers on
-      // s4, norm parts on s5), so the caller may release the workspace once its own stream has passed
-      // this point.  If the join itself cannot be enqueued, the library streams are drained on the host.
-      const hipStream_t lib_streams[4] = {s2, s3, s4, s5};
+      // that was queued on the library streams (prepares on s2, markers on s4, norm parts on s5), so the
+      // caller may release the workspace once its own stream has passed this point.  If the join
+      // itself cannot be enqueued, the library streams are drained on the host.
+      const hipStream_t lib_streams[3] = {s2, s4, s5};
       bool joined = true;
-      for (int j = 0; j < 4; ++j) {
-        if (j == 2 && !beside) continue;                    // s4 carries work only with markers beside
-        if (j == 3 && !nparts) continue;                    // s5 only with the norm by parts
+      for (int j = 0; j < 3; ++j) {
+        if (j == 0 && rc == KAIROS_GDN_OK) continue;        // the last recurrence part waited for the prepares
+        if (j == 1 && !beside) continue;                    // s4 carries work only with markers beside
+        if (j == 2 && !nparts) continue;                    // s5 only with the norm by parts
         const hipEvent_t e = ev[3 * kMaxParts + j];
         if (hipEventRecord(e, lib_streams[j]) != hipSuccess || hipStreamWaitEvent(s, e, 0) != hipSuccess)
           joined = false;
       }
       if (!joined) {
-        for (int j = 0; j < 4; ++j) (void)hipStreamSynchronize(lib_streams[j]);
+        for (int j = 0; j < 3; ++j) (void)hipStreamSynchronize(lib_streams[j]);
         if (rc == KAIROS_GDN_OK) rc = fail(KAIROS_GDN_EHIP, "joining the pipelined forward's streams failed");
       }
       if (epi_done) *epi_done = nparts && rc == KAIROS_GDN_OK;
