@@ -37,6 +37,15 @@
 // above give each such group 16 distinct 16-byte bank positions (w, q: position lg ^ lc; the 128-byte
 // rows: 8 (lc % 2) + (lg ^ lc / 2)), and they do not change under the tiles' row offsets 4 x + 32 p.
 // o is computed transposed, so each lane stores 4 consecutive columns of one token.
+//
+// What bounds a step (5.8k cycles, 2.5 us; 1.7k of them a SIMD's products): the compute waves' half before
+// B2 (u 0.8k, the state products 1.4k, their LDS reads 18 cycles each) and after it the loaders, whose 64 KB of w
+// and q take 2.8k to arrive (10 bytes a clock and issuing wave at best).  One compute wave per SIMD issues in
+// order, so operand reads go out one per product two steps ahead (in batches they added to the products: the
+// state products 2.1k), the update's tiles alternate in pairs (a product that needs the one before it waits for it:
+// update 1.4k with o in series before it, 1.7k with o inside it), and a loader forms the gates of a chunk
+// once (1.7k between B2 and the update, now 0.5k).  T = 4095 with 20 heads 227 -> 212 us, T = 32760 with 5
+// heads 1310 -> 1193.
 #include <type_traits>
 
 #include <cstdlib>
@@ -275,6 +284,8 @@ __global__ __launch_bounds__(NT_F + FL * WAVE) void wide_fused_kernel(WideFusedA
   __shared__ __align__(16) float s_qs[2 * C];             // rstd of the q rows (the in-op L2 norm)
   __shared__ __align__(16) bf16 s_o[C * C];               // the chunk's o tile [64 t][64 columns]
   __shared__ __align__(16) float s_pf[WAVE];              // landing words of the L2 prefetch
+  __shared__ __align__(16) float s_t[C];                  // exp(g_last - gc), zero past the chunk's end
+  __shared__ __align__(16) float s_f[C];                  // exp(gc), with the in-op L2 norm times rstd of the q row
   constexpr uint32_t QOFF = C * FK * 2, ABUF = C * C * 2, GBUF = C * 4;
 
   const int nvt = V / FVT, H = a.H;
@@ -356,8 +367,10 @@ __global__ __launch_bounds__(NT_F + FL * WAVE) void wide_fused_kernel(WideFusedA
     // per 128-byte line into a scratch LDS word (never read), so that the tile loads a step later
     // hit L2 instead of waiting for HBM.  The V tiles of a head share the XCD's L2, so each workgroup
     // touches a quarter of the lines: rows 16 (vt % 4) .. + 15 of w and q, lines 64 (vt % 4) .. + 63
-    // of k^T, 16 lines of Aqk.  The address unit works per line, so a full prefetch per workgroup
-    // would cost as much of it as the tile loads themselves.
+    // of k^T, 16 lines of Aqk.  The address unit works per line (4 cycles each), so a full prefetch per
+    // workgroup would cost as much of it as the tile loads themselves.  (A step of 5.8k cycles takes 7.9k
+    // without it; eighths, the head having eight tiles, 5.6k where a head's tiles share an XCD, but a head
+    // split over two leaves half its lines out: 1519 against 1493 us for 512 chunks of 20 heads.)
     const uint32_t pf_lds = lds_u32(s_pf);
     const int pf_q = (vt0 / FVT) & 3;
     auto prefetch = [&](int64_t c, int64_t t0, int nv) {     // one load per loader wave (kRc: loaders 0, 2)
@@ -579,6 +592,13 @@ __global__ __launch_bounds__(NT_F + FL * WAVE) void wide_fused_kernel(WideFusedA
       small(c_first + in, bos + in * C, chunk_nv(in), B ^ 1u);
       // the window of chunk it + 2 (convolved after B2 of step it + 1)
       const int nwin = (cvm && it + 2 < ie) ? kConvW + 1 : 0;
+      // the second half's gates, one token per lane: a wave's 64 exponentials cost one instruction here and
+      // sixteen in each compute wave, whose lanes hold sixteen tokens
+      if (lw == 3) {
+        const float* sg = s_g + B * C;
+        s_t[l] = l < chunk_nv(it) ? gexp(sg[chunk_nv(it) - 1] - sg[l]) : 0.f;
+        if constexpr (!kRc) s_f[l] = gexp(sg[l]) * (qn ? s_qs[B * C + l] : 1.f);
+      }
       if (nwin) conv_issue(w_next, it + 2);
 
       // this wave's k^T loads landed; the later ones (6 + gc / beta + the prefetch) stay in flight
@@ -691,6 +711,9 @@ __global__ __launch_bounds__(NT_F + FL * WAVE) void wide_fused_kernel(WideFusedA
     const float* sg = s_g + B * C;
     const float* sb = s_b + B * C;
 
+    Frag<bf16> wa[3][4], qa[3][4];
+    auto read_w = [&](int ks, int tm, Frag<bf16>& f) { f = ld128(A.wq[ks & 3], 256u * (ks >> 2) + rowa_off(tm, 512)); };
+    auto read_q = [&](int ks, int tm, Frag<bf16>& f) { f = ld128(A.wq[ks & 3], QOFF + 256u * (ks >> 2) + rowa_off(tm, 512)); };
     // u = Ai bf16(beta v) (wy_fast.py:55-81), rounded to bf16 as the reference stores it, from tiles
     // already in LDS at B1: the v tile is read transposed (rows s = 32 ks + 8 lg + e) and scaled by
     // beta per row.  -bf16(u) starts the w h accumulators, so they end as w h - u = -v'.
@@ -718,6 +741,13 @@ __global__ __launch_bounds__(NT_F + FL * WAVE) void wide_fused_kernel(WideFusedA
           if (ks <= tm / 2) mma(acc[tm], ld128(A.ar[ks], AI_OFF + B * ABUF + rowa_off(tm, 128)), vb[ks]);
       }
 #pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int tm = 0; tm < 4; ++tm) {
+          read_w(ks, tm, wa[ks][tm]);
+          if constexpr (!kRc) read_q(ks, tm, qa[ks][tm]);
+        }
+#pragma unroll
       for (int tm = 0; tm < 4; ++tm)
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[tm][j] = -(float)(bf16)acc[tm][j];
@@ -725,119 +755,109 @@ __global__ __launch_bounds__(NT_F + FL * WAVE) void wide_fused_kernel(WideFusedA
 
     // w h - u (rows t in the paired order, this wave's columns) and o_inter^T = h^T q^T (rows =
     // columns, cols = t = rowA(tn, lc)), with h = bf16(S) packed per 32-deep step as the B (w h)
-    // and A (h^T q^T) operand; operand reads one step ahead of the products
-    Frag<bf16> wa[2][4], qa[2][4];
-    auto read_wq = [&](int ks, Frag<bf16>(&w4)[4], Frag<bf16>(&q4)[4]) {
-      const uint32_t ra = A.wq[ks & 3];
-      const uint32_t o8 = 256u * (ks >> 2);
-#pragma unroll
-      for (int tm = 0; tm < 4; ++tm) {
-        w4[tm] = ld128(ra, o8 + rowa_off(tm, 512));
-        if constexpr (!kRc) q4[tm] = ld128(ra, QOFF + o8 + rowa_off(tm, 512));
-      }
-    };
-    read_wq(0, wa[0], qa[0]);
+    // and A (h^T q^T) operand.  One wave per SIMD issues in order, and a batch of LDS reads holds the
+    // next products back by its whole length (about 18 cycles a read, a product 16): so the reads of
+    // step ks + 2 and the packing of h for ks + 1 go out one at a time between the products of ks.
+    Frag<bf16> hb[2];
+    hb[0] = pack_acc(S[0], S[1]);
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
-      if (ks + 1 < 8) read_wq(ks + 1, wa[(ks + 1) & 1], qa[(ks + 1) & 1]);
-      __builtin_amdgcn_sched_barrier(0);
-      const Frag<bf16> hb = pack_acc(S[2 * ks], S[2 * ks + 1]);
+      if (ks + 1 < 8) hb[(ks + 1) & 1] = pack_acc(S[2 * ks + 2], S[2 * ks + 3]);
 #pragma unroll
       for (int tm = 0; tm < 4; ++tm) {
-        if constexpr (!kRc) mma(oi[tm], hb, qa[ks & 1][tm]);
-        mma(acc[tm], wa[ks & 1][tm], hb);
-      }
-      if constexpr (kRc) {                                // the snapshot: rows 32 ks + 8 lg + 4 x + j
+        if (ks + 2 < 8) read_w(ks + 2, tm, wa[(ks + 2) % 3][tm]);
+        mma(acc[tm], wa[ks % 3][tm], hb[ks & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (!kRc) {
+          if (ks + 2 < 8) read_q(ks + 2, tm, qa[(ks + 2) % 3][tm]);
+          mma(oi[tm], hb[ks & 1], qa[ks % 3][tm]);
+          __builtin_amdgcn_sched_barrier(0);
+        } else {                                          // the snapshot: rows 32 ks + 8 lg + 2 tm, + 1
 #pragma unroll
-        for (int x = 0; x < 2; ++x)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) lds_st16(snap_w, 128u * (32 * ks + 4 * x + j), hb.v[4 * x + j]);
+          for (int j = 0; j < 2; ++j)
+            lds_st16(snap_w, 128u * (32 * ks + 2 * tm + j), hb[ks & 1].v[2 * tm + j]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
-      __builtin_amdgcn_sched_barrier(0);
     }
-    f_barrier();                                          // B2: k^T in LDS; w and q tiles free
-
-    // the output's LDS operands first (one latency for all): Aqk row pieces, exp(gc_t) per tile and
-    // with the in-op L2 norm rstd of q row t
+    // the output's Aqk row pieces, in LDS already, ahead of the barrier
     Frag<bf16> aq[6];
-    float egt[4], qst[4];
     if constexpr (!kRc) {
 #pragma unroll
-      for (int tn = 0, f = 0; tn < 4; ++tn) {
-        egt[tn] = sg[32 * (tn >> 1) + 4 * (tn & 1) + ra0];
-        qst[tn] = qn ? s_qs[B * C + 32 * (tn >> 1) + 4 * (tn & 1) + ra0] : 1.f;
+      for (int tn = 0, f = 0; tn < 4; ++tn)
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks)
           if (ks <= tn / 2) aq[f++] = ld128(A.ar[ks], B * ABUF + rowa_off(tn, 128));
-      }
     }
-    // v' = u - w h (rows t = 32 (tm / 2) + 8 lg + 4 (tm % 2) + j), its bf16 value and the gated form
-    const float gl = sg[nv - 1];
-    f32x4 Y[4], Yg[4];
+    const float eg = gexp(sg[nv - 1]);
+    f_barrier();                                          // B2: k^T in LDS; w and q tiles free
+    Frag<bf16> ka[3][2][2];                               // two tiles per group, read two groups ahead
+    auto read_k = [&](int g, int x, int ks, Frag<bf16>& f) { f = ld128(A.kr[ks], rowa_off(2 * g + x, 128)); };
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) read_k(g, x, ks, ka[g][x][ks]);
+    f32x4 gt[4];
+    float fo[4];
 #pragma unroll
     for (int tm = 0; tm < 4; ++tm) {
-      Y[tm] = -acc[tm];
-      const int tr = 32 * (tm >> 1) + 8 * lg + 4 * (tm & 1);
-      const f32x4 g4 = *reinterpret_cast<const f32x4*>(sg + tr);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) Yg[tm][j] = tr + j < nv ? Y[tm][j] * gexp(gl - g4[j]) : 0.f;
+      gt[tm] = *reinterpret_cast<const f32x4*>(s_t + 32 * (tm >> 1) + 8 * lg + 4 * (tm & 1));
+      fo[tm] = kRc ? 0.f : s_f[32 * (tm >> 1) + 4 * (tm & 1) + ra0];
     }
+    S[0] *= eg;
+    S[1] *= eg;
+    // v' = -acc: its bf16 value and the gated form
     Frag<bf16> vf[2], vg[2];
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
-      vf[ks] = pack_acc(Y[2 * ks], Y[2 * ks + 1]);
-      vg[ks] = pack_acc(Yg[2 * ks], Yg[2 * ks + 1]);
+      vf[ks] = pack_acc(-acc[2 * ks], -acc[2 * ks + 1]);
+      vg[ks] = pack_acc(-acc[2 * ks] * gt[2 * ks], -acc[2 * ks + 1] * gt[2 * ks + 1]);
     }
     if constexpr (kRc) {                                  // v_new = bf16(v') into the o tile
 #pragma unroll
       for (int tm = 0; tm < 4; ++tm)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          lds_st16(vn_w[j >> 1], 128u * (32 * (tm >> 1) + 4 * (tm & 1) + j), (bf16)Y[tm][j]);
-    } else {
-    // o^T = (o_inter^T exp(gc_t) + v'^T Aqk^T) scale; lane: columns 16 w + 4 lg .. + 3 of token
-    // rowA(tn, lc), into the LDS o tile (the loader waves store it after the next B1)
-    f32x4 r[4];
-#pragma unroll
-    for (int tn = 0, f = 0; tn < 4; ++tn) {
-      r[tn] = oi[tn] * (gexp(egt[tn]) * qst[tn]);
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
-        if (ks <= tn / 2) mma(r[tn], vf[ks], aq[f++]);
+          lds_st16(vn_w[j >> 1], 128u * (32 * (tm >> 1) + 4 * (tm & 1) + j), vf[tm >> 1].v[4 * (tm & 1) + j]);
     }
+    // o^T = (o_inter^T exp(gc_t) + v'^T Aqk^T) scale; lane: columns 16 w + 4 lg .. + 3 of token
+    // rowA(tn, lc), into the LDS o tile (the loader waves store it after the next B1).  The products go
+    // first; the rest of it fills the update's products.
+    f32x4 r[4];
+    if constexpr (!kRc) {
 #pragma unroll
-    for (int tn = 0; tn < 4; ++tn) {
+      for (int tn = 0, f = 0; tn < 4; ++tn) {
+        r[tn] = oi[tn] * fo[tn];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+          if (ks <= tn / 2) mma(r[tn], vf[ks], aq[f++]);
+      }
+    }
+    auto put_o = [&](int tn) {
       const int t = 32 * (tn >> 1) + 4 * (tn & 1) + ra0;
       const f32x4 x = r[tn] * a.scale;
-      const u32x2 ov = {
-          (uint32_t)__builtin_bit_cast(uint16_t, (bf16)x[0]) | ((uint32_t)__builtin_bit_cast(uint16_t, (bf16)x[1]) << 16),
-          (uint32_t)__builtin_bit_cast(uint16_t, (bf16)x[2]) | ((uint32_t)__builtin_bit_cast(uint16_t, (bf16)x[3]) << 16)};
+      const bf16x4 ov = {(bf16)x[0], (bf16)x[1], (bf16)x[2], (bf16)x[3]};
       *reinterpret_cast<lds_u32x2*>(reinterpret_cast<lds_b*>(o_lds) + 128 * t + 16 * ((2 * wid + (lg >> 1)) ^ swz_o(t)) +
-                                    8 * (lg & 1)) = ov;
-    }
-    }
-    // S = exp(g_last) S + k^T (v' exp(g_last - gc)), pipelined like the products above
-    const float eg = gexp(gl);
-    Frag<bf16> ka[2][4][2];
-    auto read_k = [&](int k4, Frag<bf16>(&k8)[4][2]) {
-#pragma unroll
-      for (int qq = 0; qq < 4; ++qq) {
-        k8[qq][0] = ld128(A.kr[0], rowa_off(k4 + qq, 128));
-        k8[qq][1] = ld128(A.kr[1], rowa_off(k4 + qq, 128));
-      }
+                                    8 * (lg & 1)) = __builtin_bit_cast(u32x2, ov);
     };
-    read_k(0, ka[0]);
+    // S = exp(g_last) S + k^T (v' exp(g_last - gc)): the two tiles of a group alternate, so that no product
+    // waits for the one before it, and the next group is scaled between them
 #pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4) {
-      if (g4 + 1 < 4) read_k(4 * (g4 + 1), ka[(g4 + 1) & 1]);
-      __builtin_amdgcn_sched_barrier(0);
+    for (int g = 0; g < 8; ++g) {
 #pragma unroll
-      for (int qq = 0; qq < 4; ++qq) {
-        S[4 * g4 + qq] *= eg;
-        mma(S[4 * g4 + qq], ka[g4 & 1][qq][0], vg[0]);
-        mma(S[4 * g4 + qq], ka[g4 & 1][qq][1], vg[1]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+          if (g + 2 < 8) read_k(g + 2, x, ks, ka[(g + 2) % 3][x][ks]);
+          mma(S[2 * g + x], ka[g % 3][x][ks], vg[ks]);
+          if (ks == 0 && g + 1 < 8) S[2 * g + 2 + x] *= eg;
+          if constexpr (!kRc) {
+            if (g < 4 && ks == 1 && x == 0) put_o(g);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
     }
   };
 
