@@ -140,11 +140,12 @@ size_t kairos_gdn_chunk_fwd_gated_norm_workspace_size(int64_t B, int64_t T, int6
  * counterpart in the reference: it is for callers that cannot allocate (code
  * under HIP graph
  * capture, tight serving loops, harnesses that forbid allocation).  A problem
- * whose kairos_gdn_chunk_fwd_workspace_size() exceeds the array is rejected
- * with KAIROS_GDN_EWORKSPACE.  Every call on one GPU shares that GPU's array:
+ * whose scratch exceeds the array is rejected with KAIROS_GDN_EWORKSPACE (varlen
+ * batches whose kairos_gdn_chunk_fwd_workspace_size() does, but which fit with
+ * fewer, longer segments, run with those).  Every call on one GPU shares that GPU's array:
  * calls that overlap on one GPU (concurrent streams or threads) race and must
  * be serialised by the caller.  Same results as kairos_gdn_chunk_fwd (same
- * kernels); calls made through it are not recorded by the timing hook. */
+ * kernels and, but for those batches, the same segments); calls made through it are not recorded by the timing hook. */
 int kairos_gdn_chunk_fwd_noalloc(const void* q, const void* k, const void* v, const void* g, const void* beta,
                                  const float* q_scale, const float* k_scale, const void* initial_state, void* o,
                                  float* final_state, const int64_t* cu_seqlens, int64_t n_seqs, int64_t B,

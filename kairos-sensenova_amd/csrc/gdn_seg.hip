@@ -237,6 +237,38 @@ __device__ __forceinline__ SegLoc locate_seg(int s, const SegGeom& G) {
   return r;
 }
 
+// The segment s and head h of a workgroup of the (segment, head) grid.  Fixed-length batches have equal
+// segments and take them as they come.  In a varlen batch (of at most 64 sequences) a sequence's last
+// segment may be short: workgroups, which start in order of their linear index, take all heads of the full
+// segments first, then the last ones by falling length, so that the plan may hold more segments than
+// CUs (plan_segments) and the short ones fill in behind the full ones.
+__device__ __forceinline__ SegLoc pick_seg(const SegGeom& G, int& s, int& h) {
+  if (G.cu == nullptr || G.N > WAVE) {
+    s = blockIdx.x;
+    h = blockIdx.y;
+    return locate_seg(s, G);
+  }
+  const int id = blockIdx.y * gridDim.x + blockIdx.x, rank = id / G.H, l = lane_id();
+  h = id % G.H;
+  const int nc = l < G.N ? G.chunk_off[l + 1] - G.chunk_off[l] : 0;     // one sequence per lane
+  const int full = nc / G.L, rem = nc - full * G.L;
+  int before = 0, total = 0, longer = 0;
+  for (int i = 0; i < G.N; ++i) {
+    const int fi = __builtin_amdgcn_readlane(full, i), ri = __builtin_amdgcn_readlane(rem, i);
+    before += i < l ? fi : 0;
+    total += fi;
+    longer += ri > rem || (ri == rem && i < l) ? 1 : 0;
+  }
+  const uint64_t m = rank < total ? __ballot(before <= rank && rank < before + full)
+                                  : __ballot(rem > 0 && longer == rank - total);
+  SegLoc r;
+  r.ok = false;
+  if (m == 0) return r;
+  const int n = __builtin_ctzll(m);
+  s = G.seg_off[n] + (rank < total ? rank - __builtin_amdgcn_readlane(before, n) : __builtin_amdgcn_readlane(full, n));
+  return locate_seg(s, G);
+}
+
 // ---------------------------------------------------------------------------
 // LDS layouts
 // ---------------------------------------------------------------------------
@@ -1395,9 +1427,9 @@ __global__ __launch_bounds__((OutPlan<TQ, K, V>::NT)) void seg_out_kernel(SegOut
   constexpr int LDW = P::LDW, LDQ = P::LDQ, LDU = P::LDU;
   extern __shared__ __align__(16) unsigned char smem[];
 
-  const int h = blockIdx.y;
   const int H = G.H;
-  const SegLoc sl = locate_seg(blockIdx.x, G);
+  int seg, h;
+  const SegLoc sl = pick_seg(G, seg, h);
   if (!sl.ok) return;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const bool consumer = wid < P::NCW;
@@ -1455,7 +1487,7 @@ __global__ __launch_bounds__((OutPlan<TQ, K, V>::NT)) void seg_out_kernel(SegOut
 #pragma unroll
           for (int j = 0; j < 4; ++j) S[tt][ct][j] = (float)p[(16 * tt + j) * V + 16 * ct];
     } else if (sl.j > 0) {
-      const float* p = a.s_init + ((int64_t)blockIdx.x * H + h) * K * V + lane_off;
+      const float* p = a.s_init + ((int64_t)seg * H + h) * K * V + lane_off;
 #pragma unroll
       for (int tt = 0; tt < KT; ++tt)
 #pragma unroll
@@ -1854,9 +1886,9 @@ __global__ __launch_bounds__((Eng<TQ, K, V>::NT)) void seg_trans_fp8_kernel(SegT
   constexpr int NW = E::NW, NT = E::NT, KT = K / 16, KS = K / 32, CT = 2;
   extern __shared__ __align__(16) unsigned char smem[];
 
-  const int h = blockIdx.y;
   const int H = G.H;
-  const SegLoc sl = locate_seg(blockIdx.x, G);
+  int seg, h;
+  const SegLoc sl = pick_seg(G, seg, h);
   if (!sl.ok || sl.j == sl.nseg - 1) return;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int l = lane_id();
@@ -1957,7 +1989,7 @@ __global__ __launch_bounds__((Eng<TQ, K, V>::NT)) void seg_trans_fp8_kernel(SegT
     if (ci + 1 < sl.nch) step(std::integral_constant<int, 1>{}, ci + 1);
   }
 
-  const int64_t s = blockIdx.x;
+  const int64_t s = seg;
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) {
     const int c0 = 16 * ctile[ct];
@@ -2054,9 +2086,9 @@ __global__ __launch_bounds__((TransPlan<K, V>::NT)) void seg_trans_kernel(SegTra
   constexpr int KT = P::KT, KS = P::KS, CT = P::CT, NW = P::NW;
   extern __shared__ __align__(16) unsigned char smem[];
 
-  const int h = blockIdx.y;
   const int H = G.H;
-  const SegLoc sl = locate_seg(blockIdx.x, G);
+  int seg, h;
+  const SegLoc sl = pick_seg(G, seg, h);
   if (!sl.ok || sl.j == sl.nseg - 1) return;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int l = lane_id();
@@ -2218,7 +2250,7 @@ __global__ __launch_bounds__((TransPlan<K, V>::NT)) void seg_trans_kernel(SegTra
     }
   }
 
-  const int64_t s = blockIdx.x;
+  const int64_t s = seg;
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) {
     const int c0 = 16 * ctile[ct];

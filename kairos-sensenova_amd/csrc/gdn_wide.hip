@@ -42,8 +42,8 @@
 // B2 (u 0.8k, the state products 1.4k, their LDS reads 18 cycles each) and after it the loaders, whose 64 KB of w
 // and q take 2.8k to arrive (10 bytes a clock and issuing wave at best).  One compute wave per SIMD issues in
 // order, so operand reads go out one per product two steps ahead (in batches they added to the products: the
-// state products 2.1k), the update's tiles alternate in pairs (a product that needs the one before it waits for it:
-// update 1.4k with o in series before it, 1.7k with o inside it), and a loader forms the gates of a chunk
+// state products 2.1k), o's arithmetic stands between the update's products (1.2k with it, 1.4k without before),
+// and a loader forms the gates of a chunk
 // once (1.7k between B2 and the update, now 0.5k).  T = 4095 with 20 heads 227 -> 212 us, T = 32760 with 5
 // heads 1310 -> 1193.
 #include <type_traits>
@@ -842,8 +842,7 @@ __global__ __launch_bounds__(NT_F + FL * WAVE) void wide_fused_kernel(WideFusedA
       *reinterpret_cast<lds_u32x2*>(reinterpret_cast<lds_b*>(o_lds) + 128 * t + 16 * ((2 * wid + (lg >> 1)) ^ swz_o(t)) +
                                     8 * (lg & 1)) = __builtin_bit_cast(u32x2, ov);
     };
-    // S = exp(g_last) S + k^T (v' exp(g_last - gc)): the two tiles of a group alternate, so that no product
-    // waits for the one before it, and the next group is scaled between them
+    // S = exp(g_last) S + k^T (v' exp(g_last - gc)), the next group's tiles scaled between the products
 #pragma unroll
     for (int g = 0; g < 8; ++g) {
 #pragma unroll

@@ -678,3 +678,29 @@ def test_wide_varlen_order(lens, H, V):
         one = both(*(t[a][:, b:e] for a in names), t["h0"][n:n + 1], do[:, b:e], dht[n:n + 1], None)
         for i, (a, w) in enumerate(zip(got, one)):
             assert torch.equal(a[n:n + 1] if i in (1, 7) else a[:, b:e], w), (n, b, e, i)
+
+
+@pytest.mark.parametrize("lens", [[70], [128, 128, 1], [0, 330, 0, 65, 640, 63], [1 + 129 * (i % 3) for i in range(64)],
+                                  [(137 * i) % 331 for i in range(65)]], ids=["n1", "ties", "empty", "n64", "n65"])
+@pytest.mark.parametrize("H,K,dt", [(1, 64, "bf16"), (3, 128, "bf16"), (3, 128, "fp8")])
+def test_seg_varlen_order(lens, H, K, dt, monkeypatch):
+    """Packed sequences (up to 64) take their full segments first and then each sequence's last one by falling
+    length: with the segment length fixed, o and the final state have the bits of a call per sequence."""
+    monkeypatch.setenv("KAIROS_GDN_SEG_CHUNKS", "2")
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    x = make_inputs(1, int(cu[-1]), H, K, K, seed=len(lens) + K, n_states=len(lens))
+    t, kw = to_dev(x, "bf16"), {}
+    if dt == "fp8":
+        kw = {s: torch.full((H,), 0.01, device="cuda") for s in ("q_scale", "k_scale")}
+        t["q"], t["k"] = ((t[n].float() / 0.01).to(torch.float8_e4m3fn) for n in ("q", "k"))
+    names = ("q", "k", "v", "g", "beta")
+    call = lambda q, k, v, g, b, h0, c: kairos_gdn.chunk_gated_delta_rule(  # noqa: E731
+        q, k, v, g, b, initial_state=h0, output_final_state=True, cu_seqlens=torch.tensor(c, device="cuda"), **kw)
+    o, ht = call(*(t[n] for n in names), t["h0"], cu.tolist())
+    note(f"segment order: {len(lens)} sequences H={H} K={K} {dt}")
+    for n, (b, e) in enumerate(zip(cu[:-1], cu[1:])):
+        if e == b:
+            assert torch.equal(ht[n], t["h0"][n])
+            continue
+        o1, h1 = call(*(t[a][:, b:e] for a in names), t["h0"][n:n + 1], [0, int(e - b)])
+        assert torch.equal(o[:, b:e], o1) and torch.equal(ht[n:n + 1], h1), (n, b, e)
