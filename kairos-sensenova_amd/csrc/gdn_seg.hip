@@ -2347,21 +2347,21 @@ __device__ __forceinline__ void unroll_steps_upto(F& f, int j0, int rem) {
 }
 
 template <int K>
-__global__ __launch_bounds__(CombCfg<K>::NT) void seg_combine_kernel(SegCombineArgs a, SegGeom G, int total) {
+__global__ __launch_bounds__(CombCfg<K>::NT) void seg_combine_kernel(SegCombineArgs a, SegGeom G) {
   constexpr int NT = CombCfg<K>::NT;
   constexpr int LDS_T = CombCfg<K>::LDS_T;
   // s_S[buf][half][c][r]: half 0 = bf16 hi, 1 = bf16 lo of S[r][v0 + c]
   __shared__ __align__(16) bf16 s_S[2][2][16][LDS_T];
   const int V = a.V;
   const int nvt = V / 16;
-  // XCD-aware order: the V slices of one head run on one XCD and share M through its L2
-  const int per_xcd = gridDim.x / 8;
-  const int o_idx = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-  if (o_idx >= total) return;
-  const int unit = o_idx / nvt;
-  const int v0 = (o_idx % nvt) * 16;
   const int H = G.H;
-  const int n = unit / H, h = unit % H;
+  // The V slices of one head share M through an XCD's L2.  (Whole sequences laid over the XCDs put the
+  // longest of a varlen batch on one or two of them: nine segments of a 60-chunk sequence packed with
+  // five short ones, 20 heads, 85 us, 25 us so.)
+  int n, unit;
+  if (!spread_unit(H * nvt, n, unit)) return;
+  const int h = unit / nvt;
+  const int v0 = (unit % nvt) * 16;
   const int wid = threadIdx.x / WAVE;
   const int l = lane_id();
   const int lg = l >> 4, lc = l & 15;
@@ -2734,10 +2734,9 @@ int launch_seg_t(const SegFwdArgs& p, hipStream_t s) {
   }
   if (!mark(2)) return -1;
   if (p.run_combine) {
-    const int total = p.N * p.H * (V / 16);
-    const int cgrid = (total + 7) / 8 * 8;
+    const int cgrid = p.N * ((p.H * (V / 16) + 7) / 8 * 8);   // spread_unit
     SegCombineArgs ca{p.M, p.R, p.h0, p.h0_dtype, p.s_init, p.ht, V};
-    hipLaunchKernelGGL(seg_combine_kernel<K>, dim3(cgrid), dim3(CombCfg<K>::NT), 0, s, ca, G, total);
+    hipLaunchKernelGGL(seg_combine_kernel<K>, dim3(cgrid), dim3(CombCfg<K>::NT), 0, s, ca, G);
     if (hipGetLastError() != hipSuccess) return -1;
   }
   if (!mark(3)) return -1;

@@ -236,18 +236,13 @@ __device__ __forceinline__ void ld_tile64(const unsigned char* base, uint32_t ro
 // ---------------------------------------------------------------------------
 // which (sequence, head, value tile) a workgroup takes
 // ---------------------------------------------------------------------------
-// Workgroup b runs on XCD b % 8 and workgroups start in order of b.  The H V / 64 units of one sequence
-// are spread over the XCDs in runs, so that the value tiles of a head share an XCD's L2 (q, w, k^T, Aqk,
-// Ai) while every XCD takes part in every sequence; sequences follow each other, in a varlen batch of at
+// The H V / 64 units of one sequence are spread over the XCDs (spread_unit), so that the value tiles of a
+// head share an XCD's L2 (q, w, k^T, Aqk, Ai); sequences follow each other, in a varlen batch of at
 // most 64 the longest first, since the last one to start decides when the kernel ends.  A packed batch of
 // 24, 1, 49 and 99 chunks with 20 heads: 786 us with whole sequences laid over the XCDs (the longest held
 // by two of them, three rounds of its 99 chunks), 426 us so.
 __device__ __forceinline__ bool wide_unit(const int64_t* cu, int N, int units, int& n, int& idx) {
-  const int per_xcd = (units + 7) / 8;
-  const int j = blockIdx.x / 8;
-  idx = (blockIdx.x % 8) * per_xcd + j % per_xcd;
-  n = j / per_xcd;
-  if (idx >= units) return false;
+  if (!spread_unit(units, n, idx)) return false;
   if (cu != nullptr && N > 1 && N <= WAVE) {              // the sequence of rank n by length, one per lane
     const int l = lane_id(), lm = min(l, N - 1);
     const int64_t len = cu[lm + 1] - cu[lm];
