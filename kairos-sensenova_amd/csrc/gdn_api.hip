@@ -409,7 +409,7 @@ int wide_mark_mode() {
   return m < 0 || m > 2 ? 2 : m;
 }
 
-// The four streams (prepares, recurrence parts, markers, the per-part gated norm) and the events of
+// The three streams (prepares, markers, the per-part gated norm) and the events of
 // the current device, created on first use and kept until the process ends (a recorded event may be
 // recorded again: waits already enqueued keep the record they saw).  Call with g_aux_mu held.
 int aux_streams(hipStream_t* sp, hipStream_t* sm, hipStream_t* sn, hipEvent_t** events) {

@@ -237,6 +237,16 @@ __device__ __forceinline__ SegLoc locate_seg(int s, const SegGeom& G) {
   return r;
 }
 
+// Offset of element (r, c) of a segment's [K][K] map M: 16 x 32 tiles in the order of the MFMA's A operand
+// (lane r % 16 + 16 (c % 32 / 8), element c % 8), so that seg_combine loads an operand as 1 KB in a row.
+// (From row-major maps each load took 64 bytes of 16 rows, twice the lines for the address unit, which
+// bounds its step: four packed sequences of 25, 98, 195 and 512 chunks with 20 heads 616 -> 607 us, forward
+// and backward at 128 chunks 853 -> 839.)  Linear over multiples of 16 rows or 32 columns and over rows below 16.
+template <int K>
+__device__ __forceinline__ constexpr int map_off(int r, int c) {
+  return ((r >> 4) * (K / 32) + (c >> 5)) * 512 + 128 * ((c >> 3) & 3) + 8 * (r & 15) + (c & 7);
+}
+
 // The segment s and head h of a workgroup of the (segment, head) grid.  Fixed-length batches have equal
 // segments and take them as they come.  In a varlen batch (of at most 64 sequences) a sequence's last
 // segment may be short: workgroups, which start in order of their linear index, take all heads of the full
@@ -1875,7 +1885,7 @@ struct SegTransArgs {
   const void* v;
   const float* k_scale;
   const void* Ai;             // [chunks, H] chunk records from seg_prep
-  uint16_t* M;                // [NS, H] blocks of K x K bf16 M_hi then M_lo
+  uint16_t* M;                // [NS, H] blocks of K x K bf16 M_hi then M_lo (map_off)
   float* R;                   // [NS, H] blocks of K x V in accumulator-tile order (see seg_combine)
   int l2;                     // k is raw and the record carries its rstd (the in-op L2 norm)
 };
@@ -1995,7 +2005,7 @@ __global__ __launch_bounds__((Eng<TQ, K, V>::NT)) void seg_trans_fp8_kernel(SegT
     const int c0 = 16 * ctile[ct];
     if (c0 < K) {
       // M as the bf16 pair (hi, lo = bf16(M - hi)) that seg_combine multiplies in three bf16 products
-      bf16* ph = reinterpret_cast<bf16*>(a.M) + (s * H + h) * 2 * K * K + 4 * lg * K + c0 + lc;
+      bf16* ph = reinterpret_cast<bf16*>(a.M) + (s * H + h) * 2 * K * K + map_off<K>(4 * lg, c0 + lc);
       bf16* pl = ph + K * K;
 #pragma unroll
       for (int tt = 0; tt < KT; ++tt)
@@ -2003,8 +2013,8 @@ __global__ __launch_bounds__((Eng<TQ, K, V>::NT)) void seg_trans_fp8_kernel(SegT
         for (int j = 0; j < 4; ++j) {
           const float x = X[tt][ct][j];
           const bf16 hi = (bf16)x;
-          ph[(16 * tt + j) * K] = hi;
-          pl[(16 * tt + j) * K] = (bf16)(x - (float)hi);
+          ph[map_off<K>(16 * tt + j, 0)] = hi;
+          pl[map_off<K>(16 * tt + j, 0)] = (bf16)(x - (float)hi);
         }
     } else {
       // R in accumulator-tile order: tile (row tile tt, column tile cv) is 64 lanes x 4 floats
@@ -2256,7 +2266,7 @@ __global__ __launch_bounds__((TransPlan<K, V>::NT)) void seg_trans_kernel(SegTra
     const int c0 = 16 * ctile[ct];
     if (c0 < K) {
       // M as the bf16 pair (hi, lo = bf16(M - hi)) that seg_combine multiplies in three bf16 products
-      bf16* ph = reinterpret_cast<bf16*>(a.M) + (s * H + h) * 2 * K * K + 4 * lg * K + c0 + lc;
+      bf16* ph = reinterpret_cast<bf16*>(a.M) + (s * H + h) * 2 * K * K + map_off<K>(4 * lg, c0 + lc);
       bf16* pl = ph + K * K;
 #pragma unroll
       for (int tt = 0; tt < KT; ++tt)
@@ -2264,8 +2274,8 @@ __global__ __launch_bounds__((TransPlan<K, V>::NT)) void seg_trans_kernel(SegTra
         for (int j = 0; j < 4; ++j) {
           const float x = X[tt][ct][j];
           const bf16 hi = (bf16)x;
-          ph[(16 * tt + j) * K] = hi;
-          pl[(16 * tt + j) * K] = (bf16)(x - (float)hi);
+          ph[map_off<K>(16 * tt + j, 0)] = hi;
+          pl[map_off<K>(16 * tt + j, 0)] = (bf16)(x - (float)hi);
         }
     } else {
       // R in accumulator-tile order: tile (row tile tt, column tile cv) is 64 lanes x 4 floats
@@ -2292,7 +2302,7 @@ __global__ __launch_bounds__((TransPlan<K, V>::NT)) void seg_trans_kernel(SegTra
 // LDS, double buffered so that one barrier per step suffices.
 // ---------------------------------------------------------------------------
 struct SegCombineArgs {
-  const uint16_t* M;          // [NS, H] blocks of K x K bf16 M_hi then M_lo
+  const uint16_t* M;          // [NS, H] blocks of K x K bf16 M_hi then M_lo (map_off)
   const float* R;             // [NS, H] blocks of K x V: 16x16 tile (rt, ct) at 256 (rt V/16 + ct), lane l's
                               // elements (rows 16 rt + 4 (l/16) + jj, column 16 ct + l%16) at 4 l + jj
   const void* h0;
@@ -2312,12 +2322,11 @@ struct CombineMaps {
 template <int K>
 __device__ __forceinline__ void load_maps(CombineMaps<K>& c, const bf16* M, const float* R, int V, int r0, int v0) {
   const int l = lane_id();
-  const int lg = l >> 4, lc = l & 15;
-  const bf16* pm = M + (int64_t)(r0 + lc) * K + 8 * lg;
+  const bf16* pm = M + map_off<K>(r0, 0) + 8 * l;
 #pragma unroll
   for (int kb = 0; kb < K / 32; ++kb) {
-    c.mh[kb].v = *reinterpret_cast<const bf16x8*>(pm + 32 * kb);
-    c.ml[kb].v = *reinterpret_cast<const bf16x8*>(pm + K * K + 32 * kb);
+    c.mh[kb].v = *reinterpret_cast<const bf16x8*>(pm + map_off<K>(0, 32 * kb));
+    c.ml[kb].v = *reinterpret_cast<const bf16x8*>(pm + K * K + map_off<K>(0, 32 * kb));
   }
   c.r = *reinterpret_cast<const f32x4*>(R + ((r0 / 16) * (V / 16) + v0 / 16) * 256 + 4 * l);
 }
@@ -2613,7 +2622,7 @@ __global__ __launch_bounds__((RCfg<K, V, S>::NT)) void seg_bwd_combine_kernel(Se
         X[tt][j] = Bseg[blk(last) + (16 * tt + j) * V];
       }
   }
-  // maps of step j (hi then lo, row-major) as 16-byte units tid + NT i
+  // maps of step j (hi then lo) as 16-byte units tid + NT i
   u32x4 mcur[RC::UM], mnxt[RC::UM];
   f32x4 bcur[KT], bnxt[KT];
   auto load = [&](int j, u32x4 (&m)[RC::UM], f32x4 (&b)[KT]) {
@@ -2636,7 +2645,8 @@ __global__ __launch_bounds__((RCfg<K, V, S>::NT)) void seg_bwd_combine_kernel(Se
 #pragma unroll
     for (int i = 0; i < RC::UM; ++i) {
       const int e = 8 * (tid + RC::NT * i);              // element of [hi | lo]
-      const int half = e / RC::EM, r = (e % RC::EM) / K, c = e % K;
+      const int half = e / RC::EM, tile = e % RC::EM / 512, w = e % 512 / 8;      // map_off's order
+      const int r = 16 * (tile / (K / 32)) + w % 16, c = 32 * (tile % (K / 32)) + 8 * (w / 16);
       *reinterpret_cast<u32x4*>((half ? s_ml : s_mh) + moff<K>(r, c)) = mcur[i];
     }
     lds_barrier();
