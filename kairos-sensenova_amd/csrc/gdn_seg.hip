@@ -240,8 +240,8 @@ __device__ __forceinline__ SegLoc locate_seg(int s, const SegGeom& G) {
 // Offset of element (r, c) of a segment's [K][K] map M: 16 x 32 tiles in the order of the MFMA's A operand
 // (lane r % 16 + 16 (c % 32 / 8), element c % 8), so that seg_combine loads an operand as 1 KB in a row.
 // (From row-major maps each load took 64 bytes of 16 rows, twice the lines for the address unit, which
-// bounds its step: four packed sequences of 25, 98, 195 and 512 chunks with 20 heads 616 -> 607 us, forward
-// and backward at 128 chunks 853 -> 839.)  Linear over multiples of 16 rows or 32 columns and over rows below 16.
+// bounds its step: the combine of 512 chunks with 20 heads 29 -> 16 us, of a 60-chunk sequence beside five
+// short ones 25 -> 13.5.)  Linear over multiples of 16 rows or 32 columns and over rows below 16.
 template <int K>
 __device__ __forceinline__ constexpr int map_off(int r, int c) {
   return ((r >> 4) * (K / 32) + (c >> 5)) * 512 + 128 * ((c >> 3) & 3) + 8 * (r & 15) + (c & 7);
@@ -2388,8 +2388,8 @@ __global__ __launch_bounds__(CombCfg<K>::NT) void seg_combine_kernel(SegCombineA
   // loaded unconditionally (past the last step: the last step's maps again) so
   // that the number of loads issued after each stage is fixed and the wait for
   // a stage counts only the loads before it.  Three stages measured best (28 us
-  // at config 2 against 30 with four and 36 with five): the step is bound by the
-  // rate at which a CU takes in its 72 KB of maps, not by their latency.
+  // at config 2 from row-major maps, against 30 with four and 36 with five): the step is bound by
+  // the rate at which a CU takes in its 72 KB of maps (16 us in map_off's order).
   constexpr int NST = 3;
   const int nsteps = nseg - 1;
   const bf16* Mb = reinterpret_cast<const bf16*>(a.M);
