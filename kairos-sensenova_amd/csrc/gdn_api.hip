@@ -27,6 +27,24 @@
 #include "gdn_common.hpp"
 #include "gdn_kernels.h"
 
+namespace kgdn {
+
+// Compute units of the current device (queried once; 256, the MI355X count, without a device).
+int device_cus() {
+  static int cached = 0;
+  if (cached > 0) return cached;
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) {
+    (void)hipGetLastError();
+    cus = 256;
+  }
+  cached = cus;
+  return cached;
+}
+
+}  // namespace kgdn
+
 namespace {
 
 thread_local std::string g_last_error;
@@ -122,20 +140,6 @@ int chunk_map(const Geometry& G, const int64_t* cu, Carver& cv, const int32_t** 
 
 size_t stage_ws(int64_t n_seqs) { return n_seqs > 0 ? align_up(sizeof(int32_t) * (n_seqs + 1)) : 0; }
 
-// Compute units of the current device (queried once; 256, the MI355X count, without a device).
-int device_cus() {
-  static int cached = 0;
-  if (cached > 0) return cached;
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) {
-    (void)hipGetLastError();
-    cus = 256;
-  }
-  cached = cus;
-  return cached;
-}
-
 // Segment plan of the fused forward: L chunks per segment, chosen so that the
 // (segment, head) work items of the longest-running kernels fill the compute
 // units once (one 4-wave workgroup per CU).  KAIROS_GDN_SEG_CHUNKS overrides L.
@@ -153,7 +157,7 @@ struct SegPlan {
 // 195 and 512 chunks with 20 heads: L = 95, 240 workgroups, 749 us; L = 70, 280 workgroups, 654 us.
 SegPlan plan_segments(int64_t B, int64_t T, int64_t H, int64_t n_seqs, bool packed = false) {
   SegPlan P{1, 0, 0, false, false};
-  const int64_t cus = device_cus();
+  const int64_t cus = kgdn::device_cus();
   int64_t L_env = 0;
   if (const char* e = std::getenv("KAIROS_GDN_SEG_CHUNKS")) L_env = std::atoll(e);
   if (n_seqs == 0) {
@@ -363,7 +367,7 @@ constexpr int kMaxParts = 16;
 // heads, 512 chunks: 1306, 1343, 1347).  KAIROS_GDN_WIDE_PIPE sets P, KAIROS_GDN_WIDE_PIPE_GROWTH the growth.
 void wide_pipe_plan(int64_t nt, int64_t seq_heads, int64_t vtiles, int* parts, double* growth) {
   const int64_t items = nt * seq_heads;
-  const bool half_free = 2 * seq_heads * vtiles <= device_cus();
+  const bool half_free = 2 * seq_heads * vtiles <= kgdn::device_cus();
   *growth = half_free ? 3.0 : 1.4;
   *parts = half_free ? (items >= 1280 ? 2 : 1) : items >= 8192 ? 4 : items >= 3072 ? 2 : 1;
   if (const char* e = std::getenv("KAIROS_GDN_WIDE_PIPE")) {

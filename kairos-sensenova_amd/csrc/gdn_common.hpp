@@ -19,6 +19,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "gdn_order.hpp"
+
 namespace kgdn {
 
 constexpr int C = 64;        // chunk length (tokens)
@@ -95,19 +97,6 @@ template <> struct Frag<bf16> { bf16x8 v; };
 template <> struct Frag<float> { f32x4 lo, hi; };
 
 __device__ __forceinline__ int lane_id() { return threadIdx.x & (WAVE - 1); }
-
-// The sequence n and unit (head and column slice, the slices of a head consecutive) of a workgroup, where
-// each sequence has `units` of them and the grid is n_seqs * ceil(units / 8) * 8.  Workgroup b runs on XCD
-// b % 8 and workgroups start in order of b: the units of one sequence are spread over the XCDs in runs, so
-// that the slices of a head share an XCD's L2 while every XCD takes part in every sequence, and sequences
-// follow each other.  Successive sequences begin at successive XCDs, so that fewer units than XCDs, or a
-// remainder, don't pile up on the first ones.
-__device__ __forceinline__ bool spread_unit(int units, int& n, int& unit) {
-  const int per_xcd = (units + 7) / 8, j = blockIdx.x / 8;
-  n = j / per_xcd;
-  unit = (int)((blockIdx.x + n) % 8) * per_xcd + j % per_xcd;
-  return unit < units;
-}
 
 // Fragment of a K-contiguous LDS matrix: rows row0 + l%16, k = k0 + 8*(l/16) .. +7.
 template <typename T>

@@ -7,6 +7,8 @@
 
 namespace kgdn {
 
+int device_cus();         // compute units of the current device
+
 enum : int { DT_F32 = 0, DT_BF16 = 1, DT_F8E4M3 = 2 };
 
 // Shared addressing: fixed-length batches use (cu == nullptr, N = B, T = per-sequence

@@ -2355,6 +2355,11 @@ __device__ __forceinline__ void unroll_steps_upto(F& f, int j0, int rem) {
   }
 }
 
+// Whole heads to an XCD where a sequence has fewer heads than there are XCDs: 20 sequences of 31 chunks with
+// one head 78 -> 71 us a call, 4 short ones with 4 heads 42.6 -> 39.5.  From 8 heads on equal runs are 0.3
+// us faster: the chains of a sequence then load every XCD alike.
+__host__ __device__ constexpr bool comb_whole(int n_seqs, int H) { return n_seqs > 1 && H < kXcds; }
+
 template <int K>
 __global__ __launch_bounds__(CombCfg<K>::NT) void seg_combine_kernel(SegCombineArgs a, SegGeom G) {
   constexpr int NT = CombCfg<K>::NT;
@@ -2364,13 +2369,13 @@ __global__ __launch_bounds__(CombCfg<K>::NT) void seg_combine_kernel(SegCombineA
   const int V = a.V;
   const int nvt = V / 16;
   const int H = G.H;
-  // The V slices of one head share M through an XCD's L2.  (Whole sequences laid over the XCDs put the
-  // longest of a varlen batch on one or two of them: nine segments of a 60-chunk sequence packed with
-  // five short ones, 20 heads, 85 us, 25 us so.)
-  int n, unit;
-  if (!spread_unit(H * nvt, n, unit)) return;
-  const int h = unit / nvt;
-  const int v0 = (unit % nvt) * 16;
+  // The V slices of a head share M through an XCD's L2.  (With whole sequences laid over the XCDs the
+  // longest of a varlen batch sat on one or two of them: nine segments of a 60-chunk sequence packed with
+  // five short ones, 20 heads, 85 us, 25 us spread.)
+  const WgUnit wu = unit_of(blockIdx.x, G.N, H, nvt, comb_whole(G.N, H));
+  if (!wu.ok) return;
+  const int n = wu.seq, h = wu.head;
+  const int v0 = wu.slice * 16;
   const int wid = threadIdx.x / WAVE;
   const int l = lane_id();
   const int lg = l >> 4, lc = l & 15;
@@ -2744,7 +2749,7 @@ int launch_seg_t(const SegFwdArgs& p, hipStream_t s) {
   }
   if (!mark(2)) return -1;
   if (p.run_combine) {
-    const int cgrid = p.N * ((p.H * (V / 16) + 7) / 8 * 8);   // spread_unit
+    const int cgrid = unit_grid(p.N, p.H, V / 16, comb_whole(p.N, p.H));
     SegCombineArgs ca{p.M, p.R, p.h0, p.h0_dtype, p.s_init, p.ht, V};
     hipLaunchKernelGGL(seg_combine_kernel<K>, dim3(cgrid), dim3(CombCfg<K>::NT), 0, s, ca, G);
     if (hipGetLastError() != hipSuccess) return -1;

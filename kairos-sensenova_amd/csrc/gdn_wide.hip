@@ -236,13 +236,17 @@ __device__ __forceinline__ void ld_tile64(const unsigned char* base, uint32_t ro
 // ---------------------------------------------------------------------------
 // which (sequence, head, value tile) a workgroup takes
 // ---------------------------------------------------------------------------
-// The H V / 64 units of one sequence are spread over the XCDs (spread_unit), so that the value tiles of a
-// head share an XCD's L2 (q, w, k^T, Aqk, Ai); sequences follow each other, in a varlen batch of at
-// most 64 the longest first, since the last one to start decides when the kernel ends.  A packed batch of
-// 24, 1, 49 and 99 chunks with 20 heads: 786 us with whole sequences laid over the XCDs (the longest held
-// by two of them, three rounds of its 99 chunks), 426 us so.
-__device__ __forceinline__ bool wide_unit(const int64_t* cu, int N, int units, int& n, int& idx) {
-  if (!spread_unit(units, n, idx)) return false;
+// unit_of's order, so that the value tiles of a head share an XCD's L2 (q, w, k^T, Aqk, Ai); sequences
+// follow each other, in a varlen batch of at most 64 the longest first, since the last one to start decides
+// when the kernel ends.  A packed batch of 24, 1, 49 and 99 chunks with 20 heads: 786 us with whole
+// sequences laid over the XCDs (the longest held by two of them, three rounds of its 99 chunks), 426 us spread.
+__device__ __forceinline__ bool wide_unit(const int64_t* cu, int N, int H, int nvt, bool whole, int& n, int& h,
+                                          int& tile) {
+  const WgUnit u = unit_of(blockIdx.x, N, H, nvt, whole);
+  if (!u.ok) return false;
+  n = u.seq;
+  h = u.head;
+  tile = u.slice;
   if (cu != nullptr && N > 1 && N <= WAVE) {              // the sequence of rank n by length, one per lane
     const int l = lane_id(), lm = min(l, N - 1);
     const int64_t len = cu[lm + 1] - cu[lm];
@@ -266,7 +270,7 @@ __device__ __forceinline__ bool wide_unit(const int64_t* cu, int N, int units, i
 constexpr int kNormSpinMax = 1 << 14;
 
 template <bool kRc, bool kNorm>
-__global__ __launch_bounds__(NT_F + FL * WAVE) void wide_fused_kernel(WideFusedArgs a, int V) {
+__global__ __launch_bounds__(NT_F + FL * WAVE) void wide_fused_kernel(WideFusedArgs a, int V, int whole) {
   // LDS: w and q of the chunk (adjacent: q reads are w reads + 32 KB), k^T of the chunk, and two
   // buffer sets of the chunk's small tiles: Aqk, Ai, the v tile of the workgroup's 64 columns, gc, beta
   __shared__ __align__(16) bf16 s_wq[2 * C * FK];
@@ -284,11 +288,10 @@ __global__ __launch_bounds__(NT_F + FL * WAVE) void wide_fused_kernel(WideFusedA
   constexpr uint32_t QOFF = C * FK * 2, ABUF = C * C * 2, GBUF = C * 4;
 
   const int nvt = V / FVT, H = a.H;
-  int n, idx;
-  if (!wide_unit(a.cu, a.N, H * nvt, n, idx)) return;
-  const int h = idx / nvt;
+  int n, h, tile;
+  if (!wide_unit(a.cu, a.N, H, nvt, whole != 0, n, h, tile)) return;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), l = lane_id(), lg = l >> 4, lc = l & 15;
-  const int vt0 = __builtin_amdgcn_readfirstlane((idx % nvt) * FVT);      // the workgroup's first column
+  const int vt0 = __builtin_amdgcn_readfirstlane(tile * FVT);      // the workgroup's first column
 
   int64_t bos, eos, c_first;
   if (a.cu == nullptr) {
@@ -909,17 +912,16 @@ constexpr uint32_t PF_OFF = G_OFF + 2 * C * 4;       // landing words of the L2 
 constexpr uint32_t TOTAL = PF_OFF + WAVE * 4;
 }  // namespace dhu_lds
 
-__global__ __launch_bounds__(NT_F + FL * WAVE) void wide_dhu_kernel(BwdArgs a, int V) {
+__global__ __launch_bounds__(NT_F + FL * WAVE) void wide_dhu_kernel(BwdArgs a, int V, int whole) {
   using namespace dhu_lds;
   __shared__ __align__(16) unsigned char smem[TOTAL];
   const uint32_t base = lds_u32(smem);
 
   const int nvt = V / FVT, H = a.H;
-  int n, idx;
-  if (!wide_unit(a.cu, a.N, H * nvt, n, idx)) return;
-  const int h = idx / nvt;
+  int n, h, tile;
+  if (!wide_unit(a.cu, a.N, H, nvt, whole != 0, n, h, tile)) return;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), l = lane_id(), lg = l >> 4, lc = l & 15;
-  const int vt0 = __builtin_amdgcn_readfirstlane((idx % nvt) * FVT);
+  const int vt0 = __builtin_amdgcn_readfirstlane(tile * FVT);
 
   int64_t bos, eos, c_first;
   if (a.cu == nullptr) {
@@ -1636,8 +1638,9 @@ bool wide_dhu_supported(int compute_dtype, int K, int V) {
 int launch_wide_dhu(const BwdArgs& a, int V, hipStream_t s) {
   if (V % FVT != 0 || !a.qT || !a.wT || !a.dh || !a.dv2) return -2;
   if (a.N * a.H == 0) return 0;
-  const int grid = a.N * ((a.H * (V / FVT) + 7) / 8 * 8);   // wide_unit
-  hipLaunchKernelGGL(wide_dhu_kernel, dim3(grid), dim3(NT_F + FL * WAVE), 0, s, a, V);
+  const bool whole = whole_heads(a.N, a.H, V / FVT, device_cus(), false);
+  const int grid = unit_grid(a.N, a.H, V / FVT, whole);
+  hipLaunchKernelGGL(wide_dhu_kernel, dim3(grid), dim3(NT_F + FL * WAVE), 0, s, a, V, (int)whole);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -1657,15 +1660,16 @@ int launch_wide_dqkwg(const BwdArgs& a, int K, int V, int64_t nc_grid, hipStream
 
 int launch_wide_fused(const WideFusedArgs& a, int V, hipStream_t s) {
   if (V % FVT != 0 || a.N * a.H == 0) return -2;
-  const int grid = a.N * ((a.H * (V / FVT) + 7) / 8 * 8);   // wide_unit
+  const bool whole = whole_heads(a.N, a.H, V / FVT, device_cus(), a.it_end > 0);     // parts: a prepare beside
+  const int grid = unit_grid(a.N, a.H, V / FVT, whole);
   if (a.h_out) {
     if (!a.vn_out || a.ht || a.ngate) return -2;
-    hipLaunchKernelGGL((wide_fused_kernel<true, false>), dim3(grid), dim3(NT_F + FL * WAVE), 0, s, a, V);
+    hipLaunchKernelGGL((wide_fused_kernel<true, false>), dim3(grid), dim3(NT_F + FL * WAVE), 0, s, a, V, (int)whole);
   } else if (a.ngate) {
     if (V > 8 * FVT || a.nss == nullptr) return -2;
-    hipLaunchKernelGGL((wide_fused_kernel<false, true>), dim3(grid), dim3(NT_F + FL * WAVE), 0, s, a, V);
+    hipLaunchKernelGGL((wide_fused_kernel<false, true>), dim3(grid), dim3(NT_F + FL * WAVE), 0, s, a, V, (int)whole);
   } else {
-    hipLaunchKernelGGL((wide_fused_kernel<false, false>), dim3(grid), dim3(NT_F + FL * WAVE), 0, s, a, V);
+    hipLaunchKernelGGL((wide_fused_kernel<false, false>), dim3(grid), dim3(NT_F + FL * WAVE), 0, s, a, V, (int)whole);
   }
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
