@@ -129,13 +129,15 @@ struct Carver {
   }
 };
 
-// Build the varlen chunk map into the workspace (no-op for fixed length).
-int chunk_map(const Geometry& G, const int64_t* cu, Carver& cv, const int32_t** out, hipStream_t s) {
+// Build the varlen chunk map into the workspace (no-op for fixed length), and with recs the order in which
+// the K = 256 recurrences walk the sequences.
+int chunk_map(const Geometry& G, const int64_t* cu, Carver& cv, const int32_t** out, hipStream_t s,
+              kgdn::SeqRec* recs = nullptr) {
   *out = nullptr;
   if (!G.varlen) return KAIROS_GDN_OK;
   int32_t* off = static_cast<int32_t*>(cv.take(sizeof(int32_t) * (G.N + 1)));
   *out = off;
-  return from_launch(kgdn::launch_chunk_offsets(cu, (int)G.N, off, s), "chunk map");
+  return from_launch(kgdn::launch_chunk_offsets(cu, (int)G.N, off, recs, s), "chunk map");
 }
 
 size_t stage_ws(int64_t n_seqs) { return n_seqs > 0 ? align_up(sizeof(int32_t) * (n_seqs + 1)) : 0; }
@@ -341,6 +343,8 @@ size_t bwd_ws(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t n_s
     total += 2 * align_up(nc * H * K * kgdn::C * es);    // q^T (k^T first with rc_wide), w^T per chunk
   else if (rc_wide)
     total += align_up(nc * H * K * kgdn::C * es);        // k^T per chunk
+  if (!seg && (rc_wide || kgdn::wide_dhu_supported(cdt, (int)K, (int)V)))
+    total += align_up((size_t)n_seqs * sizeof(kgdn::SeqRec));    // the order of the sequences
   return total;
 }
 
@@ -478,8 +482,7 @@ int run_staged(const Geometry& G, const void* q, const void* k, const void* v, c
   const size_t es = cdt == KAIROS_GDN_F32 ? 4 : 2;
   const size_t tok = (size_t)(G.B * G.T * G.H);
   const int K = (int)G.K, V = (int)G.V, H = (int)G.H;
-  const int32_t* chunk_off = nullptr;
-  if (int rc = chunk_map(G, cu_seqlens, cv, &chunk_off, s)) return rc;
+  int32_t* chunk_off = G.varlen ? static_cast<int32_t*>(cv.take(sizeof(int32_t) * (G.N + 1))) : nullptr;
   float* gc = static_cast<float*>(cv.take(tok * sizeof(float)));
   void* w = cv.take(tok * K * es);
   const bool wide = use_wide_fused(cdt, qk_dtype, G.K, G.V);
@@ -505,6 +508,10 @@ int run_staged(const Geometry& G, const void* q, const void* k, const void* v, c
     vnT = cv.take((size_t)G.nc * H * V * kgdn::C * es);
   }
   const int N = (int)G.N;
+  // varlen: the state between parts is not used, its buffer holds the sequences' order
+  kgdn::SeqRec* recs = G.varlen ? reinterpret_cast<kgdn::SeqRec*>(st) : nullptr;
+  if (G.varlen)
+    if (int rc = from_launch(kgdn::launch_chunk_offsets(cu_seqlens, N, chunk_off, recs, s), "chunk map")) return rc;
   kgdn::PrepareArgs pa{};
   pa.k = k; pa.v = v; pa.g = g; pa.beta = beta; pa.k_scale = k_scale;
   pa.g_dtype = g_dtype; pa.beta_dtype = beta_dtype;
@@ -528,7 +535,7 @@ int run_staged(const Geometry& G, const void* q, const void* k, const void* v, c
   kgdn::WideFusedArgs fa{};
   fa.q = q; fa.kT = kt; fa.v = v; fa.w = w; fa.Ai = ai; fa.beta = bf; fa.gc = gc; fa.aqk = aqk;
   fa.h0 = h0; fa.h0_dtype = h0_dtype;
-  fa.cu = cu_seqlens; fa.chunk_off = chunk_off; fa.N = N; fa.T = G.T; fa.H = H;
+  fa.cu = cu_seqlens; fa.chunk_off = chunk_off; fa.recs = recs; fa.N = N; fa.T = G.T; fa.H = H;
   fa.scale = scale; fa.o = o; fa.ht = ht;
   fa.qs = qs;
   if (conv3) {
@@ -1135,15 +1142,19 @@ int kairos_gdn_chunk_bwd(const void* q, const void* k, const void* v, const void
   const SegPlan P = plan_segments(B, T, H, n_seqs);
   const bool segb = any_tokens && bwd_segmented(cdt, K, V, P);
   if (segb && P.ns > 0x7fffffff / 2) return fail(KAIROS_GDN_EINVAL, "%s: too many segments", what);
+  const bool rc_wide = !segb && bwd_rc_wide(cdt, qk_dtype, K, V, false);
+  const bool dhu_wide = !segb && wide_dhu_on(cdt, K, V);
   const int32_t* chunk_off = nullptr;
   const int32_t* seg_off = nullptr;
+  kgdn::SeqRec* recs = nullptr;
+  if (G.varlen && (rc_wide || dhu_wide)) recs = static_cast<kgdn::SeqRec*>(cv.take(G.N * sizeof(kgdn::SeqRec)));
   if (segb && G.varlen) {
     int32_t* co = static_cast<int32_t*>(cv.take(sizeof(int32_t) * (G.N + 1)));
     int32_t* so = static_cast<int32_t*>(cv.take(sizeof(int32_t) * (G.N + 1)));
     if (int rc = from_launch(kgdn::launch_seg_map(cu_seqlens, (int)G.N, P.L, co, so, s), "segment map")) return rc;
     chunk_off = co;
     seg_off = so;
-  } else if (int rc = chunk_map(G, cu_seqlens, cv, &chunk_off, s)) {
+  } else if (int rc = chunk_map(G, cu_seqlens, cv, &chunk_off, s, recs)) {
     return rc;
   }
   float* gc = static_cast<float*>(cv.take(tok * sizeof(float)));
@@ -1151,7 +1162,6 @@ int kairos_gdn_chunk_bwd(const void* q, const void* k, const void* v, const void
   void* w = cv.take(tok * K * es);
   void* dwb = cv.take(tok * K * es);
   void* dk1 = cv.take(tok * K * es);
-  const bool rc_wide = !segb && bwd_rc_wide(cdt, qk_dtype, K, V, false);
   void* uT = rc_wide ? nullptr : cv.take((size_t)G.nc * H * V * kgdn::C * es);
   void* Ai = cv.take(tok * kgdn::C * es);
   void* hs = cv.take((size_t)G.nc * H * K * V * es);
@@ -1161,7 +1171,6 @@ int kairos_gdn_chunk_bwd(const void* q, const void* k, const void* v, const void
   void* dv2 = cv.take(tok * V * es);
   void* qT = nullptr;                           // with rc_wide it holds k^T until the dv_local stage
   void* wT = nullptr;
-  const bool dhu_wide = !segb && wide_dhu_on(cdt, K, V);
   if (dhu_wide || rc_wide) qT = cv.take((size_t)G.nc * H * K * kgdn::C * es);
   if (dhu_wide) wT = cv.take((size_t)G.nc * H * K * kgdn::C * es);
   const void* qx = q;
@@ -1210,7 +1219,7 @@ int kairos_gdn_chunk_bwd(const void* q, const void* k, const void* v, const void
   ba.dvl = dvl; ba.dh = dhs; ba.dv2 = dv2; ba.dw = dwb; ba.dk1 = dk1; ba.dg1 = dg1;
   ba.dq = dq_k; ba.dk = dk_k; ba.dv = dv; ba.dg = dg; ba.db = dbeta; ba.dh0 = dh0;
   ba.rq = l2q_fold ? rq : nullptr;
-  ba.cu = cu_seqlens; ba.chunk_off = chunk_off; ba.N = N; ba.T = T; ba.H = (int)H; ba.scale = scale;
+  ba.cu = cu_seqlens; ba.chunk_off = chunk_off; ba.recs = recs; ba.N = N; ba.T = T; ba.H = (int)H; ba.scale = scale;
   ba.qT = dhu_wide ? qT : nullptr;
   ba.wT = wT;
   const int64_t nc_b = any_tokens ? G.nc : 0;
@@ -1219,7 +1228,7 @@ int kairos_gdn_chunk_bwd(const void* q, const void* k, const void* v, const void
       kgdn::WideFusedArgs fa{};
       fa.kT = qT; fa.v = v; fa.w = w; fa.Ai = Ai; fa.beta = dg1; fa.gc = gc;
       fa.h0 = initial_state; fa.h0_dtype = h0_dtype;
-      fa.cu = cu_seqlens; fa.chunk_off = chunk_off; fa.N = N; fa.T = T; fa.H = (int)H; fa.scale = scale;
+      fa.cu = cu_seqlens; fa.chunk_off = chunk_off; fa.recs = recs; fa.N = N; fa.T = T; fa.H = (int)H; fa.scale = scale;
       fa.h_out = hs; fa.vn_out = vn;
       if (int rc = from_launch(kgdn::launch_wide_fused(fa, (int)V, s), "fused recompute of h and v_new")) return rc;
     } else if (G.nc > 0 && any_tokens) {

@@ -98,6 +98,21 @@ template <> struct Frag<float> { f32x4 lo, hi; };
 
 __device__ __forceinline__ int lane_id() { return threadIdx.x & (WAVE - 1); }
 
+// op over the wave's lanes up to and with this one, of x >= 0 with op(0, x) = x: rows of 16 lanes by
+// shifts, then each row's last value onto the rows after it (DPP: no LDS round trip)
+template <typename Op>
+__device__ __forceinline__ int wave_prefix(int x, Op op) {
+  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false));    // row_shr 1, 2, 4, 8
+  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false));
+  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false));
+  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false));
+  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false));    // row_bcast 15 into rows 1, 3
+  return op(x, __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false)); // row_bcast 31 into rows 2, 3
+}
+__device__ __forceinline__ int wave_prefix_sum(int x) {
+  return wave_prefix(x, [](int a, int b) { return a + b; });
+}
+
 // Fragment of a K-contiguous LDS matrix: rows row0 + l%16, k = k0 + 8*(l/16) .. +7.
 template <typename T>
 __device__ __forceinline__ Frag<T> lds_frag(const T* base, int ld, int row0, int k0) {

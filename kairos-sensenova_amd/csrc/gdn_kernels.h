@@ -21,6 +21,12 @@ struct SeqArgs {
   int H;
 };
 
+// A sequence of a varlen batch in the order the K = 256 recurrences walk them (launch_chunk_offsets)
+struct alignas(16) SeqRec {
+  int64_t bos, eos;       // token range
+  int32_t n, c_first;     // sequence, index of its first chunk
+};
+
 constexpr int kConvW = 4;              // taps of the folded convolution (the layer's conv_size)
 
 // A projection the op convolves (short causal convolution + SiLU, taps of width 4) as it stages its
@@ -121,6 +127,7 @@ struct WideFusedArgs {
   int h0_dtype;
   const int64_t* cu;
   const int32_t* chunk_off;
+  const SeqRec* recs;     // varlen: [N] (launch_chunk_offsets)
   int N;
   int64_t T;
   int H;
@@ -247,6 +254,7 @@ struct BwdArgs {
   const float* rq;
   const int64_t* cu;
   const int32_t* chunk_off;
+  const SeqRec* recs;     // varlen, the K = 256 dh recurrence: [N] (launch_chunk_offsets)
   int N;
   int64_t T;
   int H;
@@ -375,7 +383,8 @@ struct GateArgs {
   int neg_eigval;
 };
 int launch_gates(const GateArgs& a, hipStream_t s);
-int launch_chunk_offsets(const int64_t* cu, int N, int32_t* chunk_off, hipStream_t s);
+// recs (or nullptr): the sequences longest first (up to 64 of them; more: as they come)
+int launch_chunk_offsets(const int64_t* cu, int N, int32_t* chunk_off, SeqRec* recs, hipStream_t s);
 int launch_cumsum(const void* g, int g_dtype, float* gc, const int64_t* cu, const int32_t* chunk_off, int N,
                   int64_t T, int H, int64_t nc_grid, hipStream_t s);
 

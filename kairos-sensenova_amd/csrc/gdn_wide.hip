@@ -240,25 +240,28 @@ __device__ __forceinline__ void ld_tile64(const unsigned char* base, uint32_t ro
 // follow each other, in a varlen batch of at most 64 the longest first, since the last one to start decides
 // when the kernel ends.  A packed batch of 24, 1, 49 and 99 chunks with 20 heads: 786 us with whole
 // sequences laid over the XCDs (the longest held by two of them, three rounds of its 99 chunks), 426 us spread.
-__device__ __forceinline__ bool wide_unit(const int64_t* cu, int N, int H, int nvt, bool whole, int& n, int& h,
-                                          int& tile) {
-  const WgUnit u = unit_of(blockIdx.x, N, H, nvt, whole);
-  if (!u.ok) return false;
-  n = u.seq;
-  h = u.head;
-  tile = u.slice;
-  if (cu != nullptr && N > 1 && N <= WAVE) {              // the sequence of rank n by length, one per lane
-    const int l = lane_id(), lm = min(l, N - 1);
-    const int64_t len = cu[lm + 1] - cu[lm];
-    const int chunks = (int)((len + C - 1) / C);
-    int rank = 0;
-    for (int i = 0; i < N; ++i) {
-      const int ci = __builtin_amdgcn_readlane(chunks, i);
-      rank += ci > chunks || (ci == chunks && i < l) ? 1 : 0;
-    }
-    n = __builtin_ctzll(__ballot(l < N && rank == n));
+struct WideUnit {
+  int n, h, tile;             // sequence, head, value tile
+  int64_t bos, eos, c_first;  // the sequence's token range and first chunk
+  bool ok;
+};
+template <typename Args>
+__device__ __forceinline__ WideUnit wide_unit(const Args& a, int nvt, bool whole) {
+  const WgUnit u = unit_of(blockIdx.x, a.N, a.H, nvt, whole);
+  WideUnit r{u.seq, u.head, u.slice, 0, 0, 0, u.ok};
+  if (!u.ok) return r;
+  if (a.cu == nullptr) {
+    r.bos = (int64_t)r.n * a.T;
+    r.eos = r.bos + a.T;
+    r.c_first = (int64_t)r.n * ((a.T + C - 1) / C);
+  } else {
+    const SeqRec rec = a.recs[u.seq];
+    r.n = rec.n;
+    r.bos = rec.bos;
+    r.eos = rec.eos;
+    r.c_first = rec.c_first;
   }
-  return true;
+  return r;
 }
 
 // kRc: the backward's recompute of the forward (chunk_delta_h.py:52-224 alone): the state before each
@@ -288,21 +291,13 @@ __global__ __launch_bounds__(NT_F + FL * WAVE) void wide_fused_kernel(WideFusedA
   constexpr uint32_t QOFF = C * FK * 2, ABUF = C * C * 2, GBUF = C * 4;
 
   const int nvt = V / FVT, H = a.H;
-  int n, h, tile;
-  if (!wide_unit(a.cu, a.N, H, nvt, whole != 0, n, h, tile)) return;
+  const WideUnit wu = wide_unit(a, nvt, whole != 0);
+  if (!wu.ok) return;
+  const int n = wu.n, h = wu.h;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), l = lane_id(), lg = l >> 4, lc = l & 15;
-  const int vt0 = __builtin_amdgcn_readfirstlane(tile * FVT);      // the workgroup's first column
+  const int vt0 = __builtin_amdgcn_readfirstlane(wu.tile * FVT);      // the workgroup's first column
 
-  int64_t bos, eos, c_first;
-  if (a.cu == nullptr) {
-    bos = (int64_t)n * a.T;
-    eos = bos + a.T;
-    c_first = (int64_t)n * ((a.T + C - 1) / C);
-  } else {
-    bos = a.cu[n];
-    eos = a.cu[n + 1];
-    c_first = a.chunk_off[n];
-  }
+  const int64_t bos = wu.bos, eos = wu.eos, c_first = wu.c_first;
   const int64_t nchunks = (eos - bos + C - 1) / C;
   // the chunks walked: ib .. ie - 1 (h0 is the state before chunk ib)
   const int64_t ib = min(a.it_begin, nchunks), ie = a.it_end > 0 ? min(a.it_end, nchunks) : nchunks;
@@ -918,21 +913,13 @@ __global__ __launch_bounds__(NT_F + FL * WAVE) void wide_dhu_kernel(BwdArgs a, i
   const uint32_t base = lds_u32(smem);
 
   const int nvt = V / FVT, H = a.H;
-  int n, h, tile;
-  if (!wide_unit(a.cu, a.N, H, nvt, whole != 0, n, h, tile)) return;
+  const WideUnit wu = wide_unit(a, nvt, whole != 0);
+  if (!wu.ok) return;
+  const int n = wu.n, h = wu.h;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), l = lane_id(), lg = l >> 4, lc = l & 15;
-  const int vt0 = __builtin_amdgcn_readfirstlane(tile * FVT);
+  const int vt0 = __builtin_amdgcn_readfirstlane(wu.tile * FVT);
 
-  int64_t bos, eos, c_first;
-  if (a.cu == nullptr) {
-    bos = (int64_t)n * a.T;
-    eos = bos + a.T;
-    c_first = (int64_t)n * ((a.T + C - 1) / C);
-  } else {
-    bos = a.cu[n];
-    eos = a.cu[n + 1];
-    c_first = a.chunk_off[n];
-  }
+  const int64_t bos = wu.bos, eos = wu.eos, c_first = wu.c_first;
   const int64_t nchunks = (eos - bos + C - 1) / C;
   const int64_t top = nchunks - 1;
   auto chunk_nv = [&](int64_t it) { return (int)min((int64_t)C, eos - (bos + it * C)); };
@@ -1636,7 +1623,7 @@ bool wide_dhu_supported(int compute_dtype, int K, int V) {
 }
 
 int launch_wide_dhu(const BwdArgs& a, int V, hipStream_t s) {
-  if (V % FVT != 0 || !a.qT || !a.wT || !a.dh || !a.dv2) return -2;
+  if (V % FVT != 0 || !a.qT || !a.wT || !a.dh || !a.dv2 || (a.cu && !a.recs)) return -2;
   if (a.N * a.H == 0) return 0;
   const bool whole = whole_heads(a.N, a.H, V / FVT, device_cus(), false);
   const int grid = unit_grid(a.N, a.H, V / FVT, whole);
@@ -1659,7 +1646,7 @@ int launch_wide_dqkwg(const BwdArgs& a, int K, int V, int64_t nc_grid, hipStream
 }
 
 int launch_wide_fused(const WideFusedArgs& a, int V, hipStream_t s) {
-  if (V % FVT != 0 || a.N * a.H == 0) return -2;
+  if (V % FVT != 0 || a.N * a.H == 0 || (a.cu && !a.recs)) return -2;
   const bool whole = whole_heads(a.N, a.H, V / FVT, device_cus(), a.it_end > 0);     // parts: a prepare beside
   const int grid = unit_grid(a.N, a.H, V / FVT, whole);
   if (a.h_out) {
