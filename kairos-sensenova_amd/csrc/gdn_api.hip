@@ -150,6 +150,7 @@ struct SegPlan {
   int nseg_fixed;     // fixed length: segments per sequence
   int64_t ns;         // segments (varlen: upper bound)
   bool trans, combine;
+  bool packed;        // varlen: the segments are taken in launch_seg_map's order
 };
 
 // A varlen batch's lengths are on the device only.  `packed` (the forward, whose kernels start full segments
@@ -158,7 +159,7 @@ struct SegPlan {
 // scratch limit that the larger plan would exceed) L such that all segments do.  Packed sequences of 25, 98,
 // 195 and 512 chunks with 20 heads: L = 95, 240 workgroups, 749 us; L = 70, 280 workgroups, 654 us.
 SegPlan plan_segments(int64_t B, int64_t T, int64_t H, int64_t n_seqs, bool packed = false) {
-  SegPlan P{1, 0, 0, false, false};
+  SegPlan P{1, 0, 0, false, false, false};
   const int64_t cus = kgdn::device_cus();
   int64_t L_env = 0;
   if (const char* e = std::getenv("KAIROS_GDN_SEG_CHUNKS")) L_env = std::atoll(e);
@@ -183,13 +184,14 @@ SegPlan plan_segments(int64_t B, int64_t T, int64_t H, int64_t n_seqs, bool pack
     return P;
   }
   const int64_t cb = T / kgdn::C + n_seqs;       // bound on the total chunk count
+  P.packed = packed && n_seqs <= 64;
   int64_t L;
   if (L_env > 0) {
     L = L_env;
   } else {
     const int64_t free_slots = std::max<int64_t>(cus - n_seqs * H, cus / 2);
     L = std::max<int64_t>(1, (cb * H + free_slots - 1) / free_slots);
-    if (packed && n_seqs <= 64) {
+    if (P.packed) {
       const int64_t per_head = std::max<int64_t>(1, cus / H);
       L = std::min(L, std::max<int64_t>(1, (cb + per_head - 1) / per_head));
     }
@@ -202,6 +204,7 @@ SegPlan plan_segments(int64_t B, int64_t T, int64_t H, int64_t n_seqs, bool pack
 
 size_t seg_ws(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t n_seqs, const SegPlan& P) {
   size_t total = n_seqs > 0 ? 2 * align_up(sizeof(int32_t) * (n_seqs + 1)) : 0;
+  if (P.packed) total += align_up(P.ns * sizeof(kgdn::SegRec));
   // chunk records: bf16 inverse [64][64] + chunk vectors, per (chunk, head)
   total += align_up((size_t)chunks_bound(B, T, n_seqs) * H * kgdn::kSegRecordBytes);
   if (P.trans || P.combine) {
@@ -850,12 +853,17 @@ static int chunk_fwd_impl(const char* what, bool profile, const void* q, const v
     return ok();
   }
   const SegPlan P = plan_segments(B, T, H, n_seqs, packed);
+  if (P.ns > 0x7fffffff / 2) return fail(KAIROS_GDN_EINVAL, "%s: too many segments", what);
   const int32_t* chunk_off = nullptr;
   const int32_t* seg_off = nullptr;
+  kgdn::SegRec* recs = nullptr;
   if (G.varlen) {
     int32_t* co = static_cast<int32_t*>(cv.take(sizeof(int32_t) * (G.N + 1)));
     int32_t* so = static_cast<int32_t*>(cv.take(sizeof(int32_t) * (G.N + 1)));
-    if (int rc = from_launch(kgdn::launch_seg_map(cu_seqlens, (int)G.N, P.L, co, so, s), "segment map")) return rc;
+    if (P.packed) recs = static_cast<kgdn::SegRec*>(cv.take(P.ns * sizeof(kgdn::SegRec)));
+    if (int rc = from_launch(kgdn::launch_seg_map(cu_seqlens, (int)G.N, P.L, co, so, recs, (int)P.ns, s),
+                             "segment map"))
+      return rc;
     chunk_off = co;
     seg_off = so;
   }
@@ -870,13 +878,12 @@ static int chunk_fwd_impl(const char* what, bool profile, const void* q, const v
     R = static_cast<float*>(cv.take(blocks * K * V * sizeof(float)));
     s_init = static_cast<float*>(cv.take(blocks * K * V * sizeof(float)));
   }
-  if (P.ns > 0x7fffffff / 2) return fail(KAIROS_GDN_EINVAL, "%s: too many segments", what);
 
   kgdn::SegFwdArgs a{};
   a.q = q; a.k = k; a.v = v; a.g = g; a.beta = beta; a.q_scale = q_scale; a.k_scale = k_scale;
   a.g_dtype = g_dtype; a.beta_dtype = beta_dtype;
   a.h0 = initial_state; a.h0_dtype = h0_dtype;
-  a.cu = cu_seqlens; a.chunk_off = chunk_off; a.seg_off = seg_off;
+  a.cu = cu_seqlens; a.chunk_off = chunk_off; a.seg_off = seg_off; a.recs = recs;
   a.N = (int)G.N; a.T = T; a.H = (int)H; a.L = P.L; a.nseg_fixed = P.nseg_fixed; a.ns_grid = P.ns;
   a.M = M; a.R = R; a.s_init = s_init; a.scale = scale; a.o = o; a.ht = final_state;
   a.Ai = Ai; a.nc_grid = nc_grid;
@@ -1151,7 +1158,9 @@ int kairos_gdn_chunk_bwd(const void* q, const void* k, const void* v, const void
   if (segb && G.varlen) {
     int32_t* co = static_cast<int32_t*>(cv.take(sizeof(int32_t) * (G.N + 1)));
     int32_t* so = static_cast<int32_t*>(cv.take(sizeof(int32_t) * (G.N + 1)));
-    if (int rc = from_launch(kgdn::launch_seg_map(cu_seqlens, (int)G.N, P.L, co, so, s), "segment map")) return rc;
+    if (int rc = from_launch(kgdn::launch_seg_map(cu_seqlens, (int)G.N, P.L, co, so, nullptr, 0, s),
+                             "segment map"))
+      return rc;
     chunk_off = co;
     seg_off = so;
   } else if (int rc = chunk_map(G, cu_seqlens, cv, &chunk_off, s, recs)) {
@@ -1314,7 +1323,7 @@ int kairos_gdn_varlen_maps(const int64_t* cu_seqlens, int64_t n_seqs, int64_t se
     return fail(KAIROS_GDN_EINVAL, "%s: seg_chunks must be in [1, 2^20]", what);
   if (!cu_seqlens || !chunk_off || !seg_off) return fail(KAIROS_GDN_EINVAL, "%s: null pointer", what);
   if (int rc = from_launch(kgdn::launch_seg_map(cu_seqlens, (int)n_seqs, (int)seg_chunks, chunk_off, seg_off,
-                                                static_cast<hipStream_t>(stream)), what))
+                                                nullptr, 0, static_cast<hipStream_t>(stream)), what))
     return rc;
   return ok();
 }

@@ -27,6 +27,15 @@ struct alignas(16) SeqRec {
   int32_t n, c_first;     // sequence, index of its first chunk
 };
 
+// A segment of a varlen batch in the order the segment scan's kernels take them (launch_seg_map)
+struct alignas(16) SegRec {
+  int32_t s, n;           // segment, its sequence
+  int32_t j, nseg;        // its index among the sequence's segments, their number
+  int32_t c0, nch;        // its first chunk within the sequence, its chunks (0: no segment)
+  int32_t cbase, pad;     // the sequence's first chunk
+  int64_t bos, eos;       // the sequence's token range
+};
+
 constexpr int kConvW = 4;              // taps of the folded convolution (the layer's conv_size)
 
 // A projection the op convolves (short causal convolution + SiLU, taps of width 4) as it stages its
@@ -188,6 +197,8 @@ struct SegFwdArgs {
   const int64_t* cu;      // varlen: [N+1] token offsets, else nullptr
   const int32_t* chunk_off;
   const int32_t* seg_off; // varlen: [N+1] segment offsets
+  const SegRec* recs;     // varlen: the segments in the order the kernels take them (launch_seg_map), or
+                          // nullptr (as they come)
   int N;
   int64_t T;
   int H;
@@ -290,7 +301,8 @@ int launch_chunk_tiles(const void* src, void* dst, int to_tiles, int elem_bytes,
 int launch_state_tiles(const void* src, void* dst, int elem_bytes, const int64_t* cu, const int32_t* chunk_off, int N,
                        int64_t T, int H, int R, int S, int64_t nc_grid, hipStream_t s);
 int launch_seg_fwd(const SegFwdArgs& a, int compute_dtype, int qk_dtype, int K, int V, hipStream_t s);
-int launch_seg_map(const int64_t* cu, int N, int L, int32_t* chunk_off, int32_t* seg_off, hipStream_t s);
+int launch_seg_map(const int64_t* cu, int N, int L, int32_t* chunk_off, int32_t* seg_off, SegRec* recs,
+                   int n_recs, hipStream_t s);
 // Segments as sequences for the stage kernels (the backward), from the geometry fields of a
 // SegFwdArgs (cu, chunk_off, seg_off, N, T, H, L, nseg_fixed, ns_grid, M):
 // seg_cu [ns_grid + 1] token and seg_coff [ns_grid + 1] chunk offsets of the segments;

@@ -194,6 +194,7 @@ struct SegGeom {
   int H;
   int L;                      // chunks per segment
   int nseg_fixed;             // fixed length: segments per sequence
+  const SegRec* recs;         // varlen: the segments in the order the workgroups take them, or nullptr
 };
 
 struct SegLoc {
@@ -248,35 +249,21 @@ __device__ __forceinline__ constexpr int map_off(int r, int c) {
 }
 
 // The segment s and head h of a workgroup of the (segment, head) grid.  Fixed-length batches have equal
-// segments and take them as they come.  In a varlen batch (of at most 64 sequences) a sequence's last
-// segment may be short: workgroups, which start in order of their linear index, take all heads of the full
-// segments first, then the last ones by falling length, so that the plan may hold more segments than
+// segments and take them as they come.  In a varlen batch a sequence's last segment may be short:
+// workgroups, which start in order of their linear index, take all heads of recs' segments in turn (the full
+// ones first, then the last ones by falling length), so that the plan may hold more segments than
 // CUs (plan_segments) and the short ones fill in behind the full ones.
 __device__ __forceinline__ SegLoc pick_seg(const SegGeom& G, int& s, int& h) {
-  if (G.cu == nullptr || G.N > WAVE) {
+  if (G.recs == nullptr) {
     s = blockIdx.x;
     h = blockIdx.y;
     return locate_seg(s, G);
   }
-  const int id = blockIdx.y * gridDim.x + blockIdx.x, rank = id / G.H, l = lane_id();
+  const int id = blockIdx.y * gridDim.x + blockIdx.x;
+  const SegRec rec = G.recs[id / G.H];
+  s = rec.s;
   h = id % G.H;
-  const int nc = l < G.N ? G.chunk_off[l + 1] - G.chunk_off[l] : 0;     // one sequence per lane
-  const int full = nc / G.L, rem = nc - full * G.L;
-  int before = 0, total = 0, longer = 0;
-  for (int i = 0; i < G.N; ++i) {
-    const int fi = __builtin_amdgcn_readlane(full, i), ri = __builtin_amdgcn_readlane(rem, i);
-    before += i < l ? fi : 0;
-    total += fi;
-    longer += ri > rem || (ri == rem && i < l) ? 1 : 0;
-  }
-  const uint64_t m = rank < total ? __ballot(before <= rank && rank < before + full)
-                                  : __ballot(rem > 0 && longer == rank - total);
-  SegLoc r;
-  r.ok = false;
-  if (m == 0) return r;
-  const int n = __builtin_ctzll(m);
-  s = G.seg_off[n] + (rank < total ? rank - __builtin_amdgcn_readlane(before, n) : __builtin_amdgcn_readlane(full, n));
-  return locate_seg(s, G);
+  return SegLoc{rec.n, rec.j, rec.nseg, rec.bos, rec.eos, rec.cbase, rec.c0, rec.nch, rec.nch > 0};
 }
 
 // ---------------------------------------------------------------------------
@@ -2490,19 +2477,44 @@ __global__ __launch_bounds__(CombCfg<K>::NT) void seg_combine_kernel(SegCombineA
   unroll_steps_upto<0, RL - 1>(step, j0, nsteps - j0);       // uniform remainder, 0 .. RL - 1 steps
 }
 
-__global__ void seg_map_kernel(const int64_t* __restrict__ cu, int N, int L, int32_t* __restrict__ chunk_off,
-                               int32_t* __restrict__ seg_off) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  int32_t ca = 0, sa = 0;
-  chunk_off[0] = 0;
-  seg_off[0] = 0;
-  for (int n = 0; n < N; ++n) {
-    const int64_t len = cu[n + 1] - cu[n];
-    const int32_t nc = (int32_t)((len + C - 1) / C);
-    ca += nc;
-    sa += (nc + L - 1) / L;
-    chunk_off[n + 1] = ca;
-    seg_off[n + 1] = sa;
+// One wave, 64 sequences at a time: chunk and segment offsets.  With recs (at most 64 sequences) also the
+// segments in the order the workgroups take them, n_recs records of which the unused ones hold no chunks.
+// (Each workgroup finding its segment among 64 sequences by itself took about 2 us in each of three kernels:
+// a training step of 64 sequences of one to nine chunks with 20 heads 1424 us so, 1339 from records.)
+__global__ __launch_bounds__(WAVE) void seg_map_kernel(const int64_t* __restrict__ cu, int N, int L,
+                                                       int32_t* __restrict__ chunk_off, int32_t* __restrict__ seg_off,
+                                                       SegRec* __restrict__ recs, int n_recs) {
+  const int l = threadIdx.x;
+  int32_t cbase = 0, sbase = 0;
+  if (l == 0) chunk_off[0] = seg_off[0] = 0;
+  for (int n0 = 0; n0 < N; n0 += WAVE) {
+    const int n = n0 + l;
+    const int64_t bos = n < N ? cu[n] : 0, eos = n < N ? cu[n + 1] : 0;
+    const int nc = (int)((eos - bos + C - 1) / C);
+    const int full = nc / L, rem = nc - full * L, ns = full + (rem > 0 ? 1 : 0);
+    const int cend = cbase + wave_prefix_sum(nc), send = sbase + wave_prefix_sum(ns);
+    if (n < N) {
+      chunk_off[n + 1] = cend;
+      seg_off[n + 1] = send;
+    }
+    if (recs != nullptr) {
+      const int fend = wave_prefix_sum(full);
+      int at = __builtin_amdgcn_readlane(fend, WAVE - 1);      // the full segments, then the others by length
+      for (int i = 0; i < N; ++i) {
+        const int ri = __builtin_amdgcn_readlane(rem, i);
+        at += ri > rem || (ri == rem && i < l) ? 1 : 0;
+      }
+      SegRec r{send - ns, n, 0, ns, 0, L, cend - nc, 0, bos, eos};
+      auto put = [&](int i) {                            // (inside the buffer whatever cu holds)
+        if ((unsigned)i < (unsigned)n_recs) recs[i] = r;
+      };
+      for (; r.j < full; ++r.s, ++r.j, r.c0 += L) put(fend - full + r.j);
+      r.nch = rem;
+      if (rem > 0) put(at);
+      for (int i = max(0, __builtin_amdgcn_readlane(send, WAVE - 1)) + l; i < n_recs; i += WAVE) recs[i] = SegRec{};
+    }
+    cbase = __builtin_amdgcn_readlane(cend, WAVE - 1);
+    sbase = __builtin_amdgcn_readlane(send, WAVE - 1);
   }
 }
 
@@ -2713,7 +2725,7 @@ int set_lds(Kern kern, size_t bytes) {
 
 template <typename TQ, int K, int V>
 int launch_seg_t(const SegFwdArgs& p, hipStream_t s) {
-  SegGeom G{p.cu, p.chunk_off, p.seg_off, p.N, p.T, p.H, p.L, p.nseg_fixed};
+  SegGeom G{p.cu, p.chunk_off, p.seg_off, p.N, p.T, p.H, p.L, p.nseg_fixed, p.recs};
   const dim3 grid((unsigned)p.ns_grid, (unsigned)p.H);
   const void* Ai = p.Ai;
   auto mark = [&](int i) { return p.events == nullptr || hipEventRecord(p.events[i], s) == hipSuccess; };
@@ -2786,7 +2798,7 @@ bool seg_fwd_supported(int compute_dtype, int K, int V) {
 }
 
 int launch_seg_seq_map(const SegFwdArgs& p, int64_t* seg_cu, int32_t* seg_coff, hipStream_t s) {
-  const SegGeom G{p.cu, p.chunk_off, p.seg_off, p.N, p.T, p.H, p.L, p.nseg_fixed};
+  const SegGeom G{p.cu, p.chunk_off, p.seg_off, p.N, p.T, p.H, p.L, p.nseg_fixed, p.recs};
   const int ns = (int)p.ns_grid;
   hipLaunchKernelGGL(seg_seq_map_kernel, dim3((unsigned)((ns + 1 + 255) / 256)), dim3(256), 0, s, G, ns, seg_cu,
                      seg_coff);
@@ -2795,7 +2807,7 @@ int launch_seg_seq_map(const SegFwdArgs& p, int64_t* seg_cu, int32_t* seg_coff, 
 
 int launch_seg_place(const SegFwdArgs& p, const void* src, int src_dtype, float* dst, int K, int V, bool first_seg,
                      hipStream_t s) {
-  const SegGeom G{p.cu, p.chunk_off, p.seg_off, p.N, p.T, p.H, p.L, p.nseg_fixed};
+  const SegGeom G{p.cu, p.chunk_off, p.seg_off, p.N, p.T, p.H, p.L, p.nseg_fixed, p.recs};
   if (p.ns_grid <= 0) return 0;
   hipLaunchKernelGGL(seg_place_kernel, dim3((unsigned)p.ns_grid, (unsigned)p.H, 8u), dim3(256), 0, s, G, src,
                      src_dtype, dst, K * V, first_seg ? 1 : 0);
@@ -2804,7 +2816,7 @@ int launch_seg_place(const SegFwdArgs& p, const void* src, int src_dtype, float*
 
 int launch_seg_bwd_combine(const SegFwdArgs& p, const float* Bseg, const float* dht, float* F, float* dh0, int K,
                            int V, hipStream_t s) {
-  const SegGeom G{p.cu, p.chunk_off, p.seg_off, p.N, p.T, p.H, p.L, p.nseg_fixed};
+  const SegGeom G{p.cu, p.chunk_off, p.seg_off, p.N, p.T, p.H, p.L, p.nseg_fixed, p.recs};
   if (p.N * p.H <= 0) return 0;
   const bf16* M = reinterpret_cast<const bf16*>(p.M);
   // V = 128: two workgroups per (sequence, head) of four waves (each reads the transposed map once
@@ -2826,8 +2838,10 @@ int launch_seg_bwd_combine(const SegFwdArgs& p, const float* Bseg, const float* 
   return -2;
 }
 
-int launch_seg_map(const int64_t* cu, int N, int L, int32_t* chunk_off, int32_t* seg_off, hipStream_t s) {
-  hipLaunchKernelGGL(seg_map_kernel, dim3(1), dim3(64), 0, s, cu, N, L, chunk_off, seg_off);
+int launch_seg_map(const int64_t* cu, int N, int L, int32_t* chunk_off, int32_t* seg_off, SegRec* recs,
+                   int n_recs, hipStream_t s) {
+  if (recs != nullptr && N > WAVE) return -2;
+  hipLaunchKernelGGL(seg_map_kernel, dim3(1), dim3(WAVE), 0, s, cu, N, L, chunk_off, seg_off, recs, n_recs);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
