@@ -156,8 +156,10 @@ size_t kairos_gdn_chunk_fwd_noalloc_max_bytes(void);
 
 /* Chunks per segment that kairos_gdn_chunk_fwd uses for this problem (the
  * segment plan: sequences are cut into segments of this many 64-token chunks
- * so that (segment, head) work items fill the GPU; the environment variable
- * KAIROS_GDN_SEG_CHUNKS overrides it).  No counterpart in the reference. */
+ * so that (segment, head) work items fill the GPU; a varlen batch of at most
+ * 64 sequences, none longer than 1.5 segments and 4 chunks, is not cut, which
+ * only the device knows; the environment variable KAIROS_GDN_SEG_CHUNKS
+ * overrides both).  No counterpart in the reference. */
 int kairos_gdn_segment_chunks(int64_t B, int64_t T, int64_t H, int64_t n_seqs);
 
 /* The varlen maps every call builds on the device from cu_seqlens (exposed for

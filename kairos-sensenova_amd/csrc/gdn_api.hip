@@ -151,6 +151,7 @@ struct SegPlan {
   int64_t ns;         // segments (varlen: upper bound)
   bool trans, combine;
   bool packed;        // varlen: the segments are taken in launch_seg_map's order
+  int whole;          // packed: no sequence is cut if the longest has at most this many chunks
 };
 
 // A varlen batch's lengths are on the device only.  `packed` (the forward, whose kernels start full segments
@@ -158,8 +159,12 @@ struct SegPlan {
 // once.  Without it (the backward, whose kernels take segments as they come; more than 64 sequences; a
 // scratch limit that the larger plan would exceed) L such that all segments do.  Packed sequences of 25, 98,
 // 195 and 512 chunks with 20 heads: L = 95, 240 workgroups, 749 us; L = 70, 280 workgroups, 654 us.
+// Cutting costs the map kernels: a sequence of m chunks in one segment takes 20 + 3.6 m us (20 + 5.5 m with
+// every CU busy), in segments of L 38 + 5.8 L (38 + 8 L).  So a packed batch whose longest sequence has at
+// most 1.5 L + 4 chunks, known on the device alone (launch_seg_map), is not cut: eight sequences of 2 to 7
+// chunks with 20 heads 52 us, 76 in segments of 4.
 SegPlan plan_segments(int64_t B, int64_t T, int64_t H, int64_t n_seqs, bool packed = false) {
-  SegPlan P{1, 0, 0, false, false, false};
+  SegPlan P{1, 0, 0, false, false, false, 0};
   const int64_t cus = kgdn::device_cus();
   int64_t L_env = 0;
   if (const char* e = std::getenv("KAIROS_GDN_SEG_CHUNKS")) L_env = std::atoll(e);
@@ -194,6 +199,7 @@ SegPlan plan_segments(int64_t B, int64_t T, int64_t H, int64_t n_seqs, bool pack
     if (P.packed) {
       const int64_t per_head = std::max<int64_t>(1, cus / H);
       L = std::min(L, std::max<int64_t>(1, (cb + per_head - 1) / per_head));
+      P.whole = (int)std::min<int64_t>((3 * L + 8) / 2, 1 << 20);
     }
   }
   P.L = (int)std::min<int64_t>(L, 1 << 20);
@@ -861,7 +867,7 @@ static int chunk_fwd_impl(const char* what, bool profile, const void* q, const v
     int32_t* co = static_cast<int32_t*>(cv.take(sizeof(int32_t) * (G.N + 1)));
     int32_t* so = static_cast<int32_t*>(cv.take(sizeof(int32_t) * (G.N + 1)));
     if (P.packed) recs = static_cast<kgdn::SegRec*>(cv.take(P.ns * sizeof(kgdn::SegRec)));
-    if (int rc = from_launch(kgdn::launch_seg_map(cu_seqlens, (int)G.N, P.L, co, so, recs, (int)P.ns, s),
+    if (int rc = from_launch(kgdn::launch_seg_map(cu_seqlens, (int)G.N, P.L, P.whole, co, so, recs, (int)P.ns, s),
                              "segment map"))
       return rc;
     chunk_off = co;
@@ -1158,7 +1164,7 @@ int kairos_gdn_chunk_bwd(const void* q, const void* k, const void* v, const void
   if (segb && G.varlen) {
     int32_t* co = static_cast<int32_t*>(cv.take(sizeof(int32_t) * (G.N + 1)));
     int32_t* so = static_cast<int32_t*>(cv.take(sizeof(int32_t) * (G.N + 1)));
-    if (int rc = from_launch(kgdn::launch_seg_map(cu_seqlens, (int)G.N, P.L, co, so, nullptr, 0, s),
+    if (int rc = from_launch(kgdn::launch_seg_map(cu_seqlens, (int)G.N, P.L, 0, co, so, nullptr, 0, s),
                              "segment map"))
       return rc;
     chunk_off = co;
@@ -1322,7 +1328,7 @@ int kairos_gdn_varlen_maps(const int64_t* cu_seqlens, int64_t n_seqs, int64_t se
   if (seg_chunks <= 0 || seg_chunks > (1 << 20))
     return fail(KAIROS_GDN_EINVAL, "%s: seg_chunks must be in [1, 2^20]", what);
   if (!cu_seqlens || !chunk_off || !seg_off) return fail(KAIROS_GDN_EINVAL, "%s: null pointer", what);
-  if (int rc = from_launch(kgdn::launch_seg_map(cu_seqlens, (int)n_seqs, (int)seg_chunks, chunk_off, seg_off,
+  if (int rc = from_launch(kgdn::launch_seg_map(cu_seqlens, (int)n_seqs, (int)seg_chunks, 0, chunk_off, seg_off,
                                                 nullptr, 0, static_cast<hipStream_t>(stream)), what))
     return rc;
   return ok();

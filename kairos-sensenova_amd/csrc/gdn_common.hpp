@@ -112,6 +112,9 @@ __device__ __forceinline__ int wave_prefix(int x, Op op) {
 __device__ __forceinline__ int wave_prefix_sum(int x) {
   return wave_prefix(x, [](int a, int b) { return a + b; });
 }
+__device__ __forceinline__ int wave_max(int x) {
+  return __builtin_amdgcn_readlane(wave_prefix(x, [](int a, int b) { return a > b ? a : b; }), WAVE - 1);
+}
 
 // Fragment of a K-contiguous LDS matrix: rows row0 + l%16, k = k0 + 8*(l/16) .. +7.
 template <typename T>

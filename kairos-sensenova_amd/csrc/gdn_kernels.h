@@ -301,7 +301,7 @@ int launch_chunk_tiles(const void* src, void* dst, int to_tiles, int elem_bytes,
 int launch_state_tiles(const void* src, void* dst, int elem_bytes, const int64_t* cu, const int32_t* chunk_off, int N,
                        int64_t T, int H, int R, int S, int64_t nc_grid, hipStream_t s);
 int launch_seg_fwd(const SegFwdArgs& a, int compute_dtype, int qk_dtype, int K, int V, hipStream_t s);
-int launch_seg_map(const int64_t* cu, int N, int L, int32_t* chunk_off, int32_t* seg_off, SegRec* recs,
+int launch_seg_map(const int64_t* cu, int N, int L, int whole, int32_t* chunk_off, int32_t* seg_off, SegRec* recs,
                    int n_recs, hipStream_t s);
 // Segments as sequences for the stage kernels (the backward), from the geometry fields of a
 // SegFwdArgs (cu, chunk_off, seg_off, N, T, H, L, nseg_fixed, ns_grid, M):

@@ -2478,10 +2478,10 @@ __global__ __launch_bounds__(CombCfg<K>::NT) void seg_combine_kernel(SegCombineA
 }
 
 // One wave, 64 sequences at a time: chunk and segment offsets.  With recs (at most 64 sequences) also the
-// segments in the order the workgroups take them, n_recs records of which the unused ones hold no chunks.
-// (Each workgroup finding its segment among 64 sequences by itself took about 2 us in each of three kernels:
-// a training step of 64 sequences of one to nine chunks with 20 heads 1424 us so, 1339 from records.)
-__global__ __launch_bounds__(WAVE) void seg_map_kernel(const int64_t* __restrict__ cu, int N, int L,
+// segments in the order the workgroups take them, n_recs records of which the unused ones hold no chunks; and
+// if the longest sequence has at most `whole` chunks, every sequence is one segment (plan_segments).
+// (Each workgroup finding its segment among 64 sequences by itself took about 2 us in each of three kernels.)
+__global__ __launch_bounds__(WAVE) void seg_map_kernel(const int64_t* __restrict__ cu, int N, int L, int whole,
                                                        int32_t* __restrict__ chunk_off, int32_t* __restrict__ seg_off,
                                                        SegRec* __restrict__ recs, int n_recs) {
   const int l = threadIdx.x;
@@ -2491,6 +2491,10 @@ __global__ __launch_bounds__(WAVE) void seg_map_kernel(const int64_t* __restrict
     const int n = n0 + l;
     const int64_t bos = n < N ? cu[n] : 0, eos = n < N ? cu[n + 1] : 0;
     const int nc = (int)((eos - bos + C - 1) / C);
+    if (recs != nullptr) {
+      const int longest = wave_max(nc);
+      if (longest <= whole) L = max(longest, 1);
+    }
     const int full = nc / L, rem = nc - full * L, ns = full + (rem > 0 ? 1 : 0);
     const int cend = cbase + wave_prefix_sum(nc), send = sbase + wave_prefix_sum(ns);
     if (n < N) {
@@ -2838,10 +2842,10 @@ int launch_seg_bwd_combine(const SegFwdArgs& p, const float* Bseg, const float* 
   return -2;
 }
 
-int launch_seg_map(const int64_t* cu, int N, int L, int32_t* chunk_off, int32_t* seg_off, SegRec* recs,
+int launch_seg_map(const int64_t* cu, int N, int L, int whole, int32_t* chunk_off, int32_t* seg_off, SegRec* recs,
                    int n_recs, hipStream_t s) {
   if (recs != nullptr && N > WAVE) return -2;
-  hipLaunchKernelGGL(seg_map_kernel, dim3(1), dim3(WAVE), 0, s, cu, N, L, chunk_off, seg_off, recs, n_recs);
+  hipLaunchKernelGGL(seg_map_kernel, dim3(1), dim3(WAVE), 0, s, cu, N, L, whole, chunk_off, seg_off, recs, n_recs);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

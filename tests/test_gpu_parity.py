@@ -704,3 +704,44 @@ def test_seg_varlen_order(lens, H, K, dt, monkeypatch):
             continue
         o1, h1 = call(*(t[a][:, b:e] for a in names), t["h0"][n:n + 1], [0, int(e - b)])
         assert torch.equal(o[:, b:e], o1) and torch.equal(ht[n:n + 1], h1), (n, b, e)
+
+
+@pytest.mark.parametrize("n,H,longest", [(8, 20, None), (8, 20, 40), (3, 4, None), (40, 20, None)],
+                         ids=["n8", "n8_long", "n3", "n40"])
+def test_packed_sequences_cut_only_where_it_pays(n, H, longest, monkeypatch):
+    """A packed batch whose longest sequence has at most 1.5 L + 4 chunks (L: the plan's segments) is not
+    cut: the bits of segments as long as that sequence.  One chunk more, and they are the bits of L."""
+    lib = kairos_gdn._lib.load()
+    K = 128
+
+    def run(lens, L=None):
+        cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+        if L is None:
+            monkeypatch.delenv("KAIROS_GDN_SEG_CHUNKS", raising=False)
+        else:
+            monkeypatch.setenv("KAIROS_GDN_SEG_CHUNKS", str(L))
+        x = make_inputs(1, int(cu[-1]), H, K, K, seed=len(lens), n_states=len(lens))
+        x["g"] *= 0.02                                 # slow decay: the state outlives a segment
+        t = to_dev(x, "bf16")
+        return kairos_gdn.chunk_gated_delta_rule(*(t[a] for a in ("q", "k", "v", "g", "beta")), initial_state=t["h0"],
+                                                 output_final_state=True, cu_seqlens=torch.from_numpy(cu).cuda())
+
+    def plan(lens):
+        monkeypatch.delenv("KAIROS_GDN_SEG_CHUNKS", raising=False)
+        return lib.kairos_gdn_segment_chunks(1, int(sum(lens)), H, len(lens))
+
+    rest = [64 * (i % 4) + 7 for i in range(n - 1)]
+    if longest is None:                                # the longest sequence that stays whole, and one chunk more
+        longest = next(m for m in range(1, 99) if 2 * (m + 1) > 3 * plan([64 * (m + 1)] + rest) + 8)
+        cases = [(longest, True), (longest + 1, False)]
+    else:
+        cases = [(longest, False)]
+    for m, whole in cases:
+        lens = [64 * m] + rest
+        L = plan(lens)
+        assert (2 * m <= 3 * L + 8) == whole and m > L
+        note(f"packed batch of {n}, H={H}: longest {m} chunks, L={L}, whole={whole}")
+        got, as_one, cut = run(lens), run(lens, m), run(lens, L)
+        assert not torch.equal(as_one[0], cut[0])
+        for a, b in zip(got, as_one if whole else cut):
+            assert torch.equal(a, b)
