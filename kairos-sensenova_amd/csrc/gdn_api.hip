@@ -26,6 +26,7 @@
 #include "../../include/kairos_gdn.h"
 #include "gdn_common.hpp"
 #include "gdn_kernels.h"
+#include "gdn_plan.hpp"
 
 namespace kgdn {
 
@@ -370,28 +371,18 @@ size_t bwd_ws(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t n_s
 // prepare's 10^4 workgroups could take every CU and hold the recurrence back).
 constexpr int kMaxParts = 16;
 
-// Parts and their growth.  A part boundary costs the caller's stream about 16 us of waits, and what it hides
-// is the prepare of the later parts (about 0.05 us per (chunk, head) on all CUs), so short calls run in one
-// part: with 20 heads 188 -> 99 us at 25 chunks and 294 -> 225 us at 64 against four parts, one and two parts
-// equal (434 us) at 128, two ahead at 256 (795 against 849, three 793, four 808) and four at 512 (1499, two
-// 1543, one 1667).  Where the recurrence takes at most half of the CUs the later prepares run on the others
-// several times faster than it walks, so the first part can be small: two parts growing by 3, from 1280
-// items on (10 heads, 128 chunks: 372 against 379 us; 512 chunks: 1353, four parts by 1.4 1371, one 1443; 5
-// heads, 512 chunks: 1306, 1343, 1347).  KAIROS_GDN_WIDE_PIPE sets P, KAIROS_GDN_WIDE_PIPE_GROWTH the growth.
-void wide_pipe_plan(int64_t nt, int64_t seq_heads, int64_t vtiles, int* parts, double* growth) {
-  const int64_t items = nt * seq_heads;
-  const bool half_free = 2 * seq_heads * vtiles <= kgdn::device_cus();
-  *growth = half_free ? 3.0 : 1.4;
-  *parts = half_free ? (items >= 1280 ? 2 : 1) : items >= 8192 ? 4 : items >= 3072 ? 2 : 1;
+// KAIROS_GDN_WIDE_PIPE sets the number of parts, KAIROS_GDN_WIDE_PIPE_GROWTH their growth.
+kgdn::PipePlan wide_pipe(int64_t nt, int64_t seq_heads, int64_t vtiles) {
+  kgdn::PipePlan p = kgdn::wide_pipe_plan(nt, seq_heads, vtiles, kgdn::device_cus());
   if (const char* e = std::getenv("KAIROS_GDN_WIDE_PIPE")) {
-    const int p = std::atoi(e);
-    *parts = p < 1 ? 1 : p > kMaxParts ? kMaxParts : p;
-    *growth = 1.4;
+    const int n = std::atoi(e);
+    p = {n < 1 ? 1 : n > kMaxParts ? kMaxParts : n, 1.4};
   }
   if (const char* e = std::getenv("KAIROS_GDN_WIDE_PIPE_GROWTH")) {
     const double g = std::atof(e);
-    *growth = g < 0.25 ? 0.25 : g > 4.0 ? 4.0 : g;
+    p.growth = g < 0.25 ? 0.25 : g > 4.0 ? 4.0 : g;
   }
+  return p;
 }
 
 // Chunk boundaries of P parts of nt chunks with sizes growing by `growth`: b[0] = 0, b[P] = nt, every
@@ -559,9 +550,9 @@ int run_staged(const Geometry& G, const void* q, const void* k, const void* v, c
   }
   if (wide && G.nc > 0 && may_fork && cu_seqlens == nullptr) {
     const int64_t nt = (G.T + kgdn::C - 1) / kgdn::C;
-    int P = 1;
-    double growth = 1.0;
-    wide_pipe_plan(nt, (int64_t)N * H, V / 64, &P, &growth);
+    const kgdn::PipePlan plan = wide_pipe(nt, (int64_t)N * H, V / 64);
+    const double growth = plan.growth;
+    int P = plan.parts;
     if (nt < 2 * P) P = 1;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (P > 1 && (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)) P = 1;

@@ -345,6 +345,27 @@ def test_model_head_dims_pipeline_parts(with_h0, monkeypatch):
         assert torch.equal(ht, ht1), (parts, growth)
 
 
+@pytest.mark.parametrize("H,V,nt", [(5, 512, 257), (10, 64, 210), (20, 512, 155), (20, 512, 410)],
+                         ids=["2x3", "4x1.4_narrow", "2x1.4", "4x1.4"])
+def test_model_head_dims_default_parts(H, V, nt, monkeypatch):
+    """Every form that the K = 256 forward takes in parts by itself (the layer's mode, a ragged last chunk): the
+    bits of one part."""
+    note(f"K=256 default parts H={H} V={V}, {nt} chunks")
+    monkeypatch.delenv("KAIROS_GDN_WIDE_PIPE", raising=False)
+    monkeypatch.delenv("KAIROS_GDN_WIDE_PIPE_GROWTH", raising=False)
+    T = 64 * nt - 27
+    gen = torch.Generator(device="cuda").manual_seed(nt)
+    r = lambda *sh: torch.randn(*sh, device="cuda", generator=gen)  # noqa: E731
+    q, k, v = (r(1, T, H, d).to(torch.bfloat16) for d in (256, 256, V))
+    beta, g, h0 = torch.sigmoid(r(1, T, H)).to(torch.bfloat16), -0.1 * r(1, T, H).abs(), 0.02 * r(1, H, 256, V)
+    run = lambda: kairos_gdn.chunk_gated_delta_rule(q, k, v, g, beta, initial_state=h0,  # noqa: E731
+                                                    output_final_state=True, use_qk_l2norm_in_kernel=True)
+    o, ht = run()
+    monkeypatch.setenv("KAIROS_GDN_WIDE_PIPE", "1")
+    o1, ht1 = run()
+    assert bool(torch.isfinite(o).all()) and torch.equal(o, o1) and torch.equal(ht, ht1)
+
+
 def test_empty_sequence_returns_initial_state():
     note("T=0")
     x = make_inputs(2, 0, 2, 64, 64, seed=1, dtype="bf16")
