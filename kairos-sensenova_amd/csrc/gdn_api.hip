@@ -763,11 +763,14 @@ static bool fused_norm_on(const NormEpilogue* epi) {
 // layer shape the folded norm makes the call slower than the forward followed by the norm kernel
 // (3.04 against 1.90 ms): the fused kernel's step is bound by its loader waves, which share the SIMDs
 // with the compute waves, and the norm adds its gate and o rows to their loads and its sigmoid and
-// scaling to their VALU issue.
-static bool wide_norm_on(const NormEpilogue* epi, int cdt, int qk_dtype, int64_t K, int64_t V) {
+// scaling to their VALU issue.  A head's workgroups wait for each other's sums, so they must all hold a CU:
+// with more workgroups than CUs some of a head's would wait for others that start when a whole sequence
+// has been walked, longer than the bounded wait allows.
+static bool wide_norm_on(const NormEpilogue* epi, int cdt, int qk_dtype, int64_t N, int64_t H, int64_t K, int64_t V) {
   const char* e = std::getenv("KAIROS_GDN_WIDE_NORM_FOLD");
   return e && e[0] == '1' && e[1] == 0 && fused_norm_on(epi) && !kgdn::seg_fwd_supported(cdt, (int)K, (int)V) &&
-         use_wide_fused(cdt, qk_dtype, K, V) && V % 64 == 0 && V <= 512;
+         use_wide_fused(cdt, qk_dtype, K, V) && V % 64 == 0 && V <= 512 &&
+         kgdn::wide_fused_resident(N, H, V);
 }
 
 // Tag of one call's exchange entries: a per-process start (time and pid) plus a call count, never 0
@@ -824,7 +827,7 @@ static int chunk_fwd_impl(const char* what, bool profile, const void* q, const v
     // the gated norm in the fused K = 256 form, given room for its exchange buffer beyond `need`
     kgdn::WideFusedArgs wn{};
     const size_t nb = kgdn::wide_norm_bytes(G.nc, H);
-    const bool wfold = any_tokens && wide_norm_on(epi, cdt, qk_dtype, K, V) && workspace_bytes >= need + nb;
+    const bool wfold = any_tokens && wide_norm_on(epi, cdt, qk_dtype, G.N, H, K, V) && workspace_bytes >= need + nb;
     if (wfold) {
       wn.ngate = epi->gate; wn.nw = epi->w; wn.nb = epi->b; wn.nw_dtype = epi->w_dtype;
       wn.neps = epi->eps; wn.nsigmoid_only = epi->sigmoid_only;
@@ -945,7 +948,7 @@ size_t kairos_gdn_chunk_fwd_gated_norm_workspace_size(int64_t B, int64_t T, int6
   if (need == 0 && (B <= 0 || T < 0 || H <= 0 || K <= 0 || V <= 0 || n_seqs < 0)) return 0;
   const int cdt = compute_dtype(qk_dtype, v_dtype);
   const NormEpilogue probe{nullptr, nullptr, nullptr, KAIROS_GDN_BF16, KAIROS_GDN_F32, 0.f, 0};
-  if (cdt < 0 || !wide_norm_on(&probe, cdt, qk_dtype, K, V)) return need;
+  if (cdt < 0 || !wide_norm_on(&probe, cdt, qk_dtype, n_seqs > 0 ? n_seqs : B, H, K, V)) return need;
   return need + kgdn::wide_norm_bytes(chunks_bound(B, T, n_seqs), H);
 }
 

@@ -169,6 +169,8 @@ struct WideFusedArgs {
 // Bytes of WideFusedArgs::nss for nc chunks of H heads
 inline size_t wide_norm_bytes(int64_t nc, int64_t H) { return (size_t)nc * H * 64 * 8 * 8 + 1024; }
 bool wide_fused_supported(int compute_dtype, int qk_dtype, int K, int V);
+// Whether the fused kernel's workgroups all hold a CU at once (its gated norm needs that)
+bool wide_fused_resident(int64_t N, int64_t H, int64_t V);
 int launch_wide_fused(const WideFusedArgs& a, int V, hipStream_t s);
 // An empty one-workgroup kernel: a point in a stream's order that an event can mark.
 int launch_marker(hipStream_t s);

@@ -268,7 +268,8 @@ __device__ __forceinline__ WideUnit wide_unit(const Args& a, int nvt, bool whole
 // chunk (bf16, through the q half of the w / q tile, which q does not use here) and v_new (through the o
 // tile) leave as whole rows stored by the loader waves; q, Aqk and the output products are skipped.
 // the gated norm's exchange: how many times a workgroup loads a share again while the other workgroups of
-// its head have not yet published it (each try a sleep of ~128 clocks and a load, ~1-2 us: ~25 ms in all);
+// its head have not yet published it (each try a sleep of ~128 clocks and a load, ~1-2 us: ~25 ms in all,
+// while all of them are resident: wide_fused_resident);
 // a share still missing then makes its token's rows NaN rather than holding the GPU
 constexpr int kNormSpinMax = 1 << 14;
 
@@ -412,7 +413,8 @@ __global__ __launch_bounds__(NT_F + FL * WAVE) void wide_fused_kernel(WideFusedA
     //      its gate row and its o row (back from L2) are loaded; in step c + 4, any share without the
     //      call's tag is loaded again until it has it, and y replaces o.  The shares travel as single
     //      8-byte agent-scope atomics, so a matching tag vouches for its value; the head's workgroups run
-    //      in step, so a share is normally in place two steps before it is loaded.  The loaders bound
+    //      in step (each holds a CU: wide_fused_resident), so a share is normally in place two steps
+    //      before it is loaded.  The loaders bound
     //      the step: everything here runs after the k^T loads are issued, while the loaders would wait
     //      for them anyway, and every memory instruction from the publication on executes on all lanes
     //      (masked rows go to a dummy line past the shares), so the counted wait before B2 stays exact.
@@ -1645,6 +1647,13 @@ int launch_wide_dqkwg(const BwdArgs& a, int K, int V, int64_t nc_grid, hipStream
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+bool wide_fused_resident(int64_t N, int64_t H, int64_t V) {
+  const int64_t cus = device_cus();
+  if (N * H * (V / FVT) > cus) return false;
+  const int n = (int)N, h = (int)H, s = (int)(V / FVT);
+  return unit_grid(n, h, s, false) <= cus && unit_grid(n, h, s, whole_heads(n, h, s, (int)cus, false)) <= cus;
+}
+
 int launch_wide_fused(const WideFusedArgs& a, int V, hipStream_t s) {
   if (V % FVT != 0 || a.N * a.H == 0 || (a.cu && !a.recs)) return -2;
   const bool whole = whole_heads(a.N, a.H, V / FVT, device_cus(), a.it_end > 0);     // parts: a prepare beside
@@ -1653,7 +1662,7 @@ int launch_wide_fused(const WideFusedArgs& a, int V, hipStream_t s) {
     if (!a.vn_out || a.ht || a.ngate) return -2;
     hipLaunchKernelGGL((wide_fused_kernel<true, false>), dim3(grid), dim3(NT_F + FL * WAVE), 0, s, a, V, (int)whole);
   } else if (a.ngate) {
-    if (V > 8 * FVT || a.nss == nullptr) return -2;
+    if (V > 8 * FVT || a.nss == nullptr || !wide_fused_resident(a.N, a.H, V)) return -2;
     hipLaunchKernelGGL((wide_fused_kernel<false, true>), dim3(grid), dim3(NT_F + FL * WAVE), 0, s, a, V, (int)whole);
   } else {
     hipLaunchKernelGGL((wide_fused_kernel<false, false>), dim3(grid), dim3(NT_F + FL * WAVE), 0, s, a, V, (int)whole);

@@ -287,3 +287,16 @@ def test_product_does_not_import_oracle():
                 text = open(os.path.join(dirpath, f)).read()
                 assert not re.search(r"^\s*(from|import)\s+oracle", text, re.M), f
                 assert "gdn_oracle" not in text, f
+
+
+def test_folded_norm_needs_every_workgroup_resident(monkeypatch):
+    """KAIROS_GDN_WIDE_NORM_FOLD=1: a head's workgroups wait for each other, so the fold runs only where all
+    workgroups hold a CU at once.  Two sequences of 20 heads (320 workgroups) need no exchange buffer."""
+    lib = _lib.load()
+    monkeypatch.setenv("KAIROS_GDN_WIDE_NORM_FOLD", "1")
+    monkeypatch.setenv("KAIROS_GDN_FUSED_NORM", "1")
+    for B, H, V, cu_n, fold in [(1, 20, 512, 0, True), (2, 20, 512, 0, False), (1, 20, 512, 2, False), (1, 32, 512, 0, True),
+                                (1, 33, 512, 0, False), (2, 16, 512, 0, True), (4, 64, 64, 0, True)]:
+        args = (B, 4096, H, 256, V, cu_n, _lib.BF16, _lib.BF16, 1)
+        extra = lib.kairos_gdn_chunk_fwd_gated_norm_workspace_size(*args) - lib.kairos_gdn_chunk_fwd_workspace_size(*args)
+        assert (extra > 0) == fold, (B, H, V, cu_n)

@@ -295,3 +295,23 @@ def test_gated_norm_argument_errors():
     with pytest.raises(ValueError, match="norm_weight must have shape"):
         kairos_gdn.chunk_gated_delta_rule_gated_norm(d["q"], d["k"], d["v"], d["g"], d["beta"], gate,
                                                      torch.ones(32, device="cuda"))
+
+
+def test_folded_norm_refused_for_two_rounds(monkeypatch):
+    """Two packed sequences of 20 heads with the fold asked for: the forward followed by the norm kernel."""
+    T, H, K, V = 200, 20, 256, 512
+    note(f"gated norm fold asked for with 320 workgroups T={T} H={H}")
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    r = lambda *sh: torch.randn(*sh, device="cuda", generator=gen)  # noqa: E731
+    q, k, v = (r(1, T, H, d).to(torch.bfloat16) for d in (K, K, V))
+    beta, g, h0 = torch.sigmoid(r(1, T, H)).to(torch.bfloat16), -r(1, T, H).abs(), 0.02 * r(2, H, K, V)
+    gate, w = r(1, T, H, V).to(torch.bfloat16), torch.linspace(0.5, 1.5, V, device="cuda")
+    cu = torch.tensor([0, 137, T], device="cuda")
+    monkeypatch.setenv("KAIROS_GDN_WIDE_NORM_FOLD", "1")
+    y, ht = kairos_gdn.chunk_gated_delta_rule_gated_norm(q, k, v, g, beta, gate, w, initial_state=h0, cu_seqlens=cu,
+                                                         output_final_state=True, use_qk_l2norm_in_kernel=True)
+    o, ht2 = kairos_gdn.chunk_gated_delta_rule(q, k, v, g, beta, initial_state=h0, output_final_state=True,
+                                               cu_seqlens=cu, use_qk_l2norm_in_kernel=True)
+    assert torch.equal(ht, ht2)
+    assert torch.equal(y.reshape(-1, V), kairos_gdn.rms_norm_gated_fwd(o.reshape(-1, V), gate.reshape(-1, V), w, None,
+                                                                       "swish", 1e-5))
