@@ -775,6 +775,15 @@ __global__ __launch_bounds__(NT_F + FL * WAVE) void wide_fused_kernel(WideFusedA
         }
       }
     }
+    // rows past the chunk's end are copies of its first, and an infinite one times their zero gate would be NaN
+    // (here, where the products end, the check is free; in the update it cost 1.5% of the step)
+    if (nv < C) {
+#pragma unroll
+      for (int tm = 0; tm < 4; ++tm)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (32 * (tm >> 1) + 8 * lg + 4 * (tm & 1) + j >= nv) acc[tm][j] = 0.f;
+    }
     // the output's Aqk row pieces, in LDS already, ahead of the barrier
     Frag<bf16> aq[6];
     if constexpr (!kRc) {

@@ -766,3 +766,22 @@ def test_packed_sequences_cut_only_where_it_pays(n, H, longest, monkeypatch):
         assert not torch.equal(as_one[0], cut[0])
         for a, b in zip(got, as_one if whole else cut):
             assert torch.equal(a, b)
+
+
+def test_wide_infinite_state(monkeypatch):
+    """K = 256, one token and a state with an infinite entry: with k > 0 the final state's other rows are
+    infinite, not NaN, as in the stage kernels (the chunk's rows past its end are copies of its first, whose
+    product with a zero gate must not reach the state)."""
+    x = make_inputs(1, 1, 2, 256, 64, seed=1)
+    x["k"] = np.abs(x["k"]) + 0.01
+    x["h0"][0, 1, 5, 3] = np.inf
+    t = to_dev(x, "bf16")
+    note("infinite state")
+    got = {}
+    for fused in ("0", "1"):
+        monkeypatch.setenv("KAIROS_GDN_WIDE_FUSED", fused)
+        got[fused] = kairos_gdn.chunk_gated_delta_rule(t["q"], t["k"], t["v"], t["g"], t["beta"],
+                                                       initial_state=t["h0"], output_final_state=True)[1].cpu()
+    assert torch.isneginf(got["0"][0, 1, :5, 3]).all() and torch.isnan(got["0"][0, 1, 5, 3])
+    for same in (torch.isnan, torch.isneginf):
+        assert bool((same(got["1"]) == same(got["0"])).all()), same.__name__
