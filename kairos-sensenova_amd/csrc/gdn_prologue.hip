@@ -20,6 +20,8 @@
 // Layout of the convolution: lane = 8 consecutive channels (one 16-byte bf16
 // load), wave = 512 channels of a run of 4 or 8 consecutive tokens, whose rows
 // and W - 1 halo rows it loads together.  Every kernel here is HBM-bound.
+#include <algorithm>
+
 #include "gdn_common.hpp"
 #include "gdn_kernels.h"
 
@@ -31,7 +33,8 @@ constexpr int kConvWaves = 4;
 // From this many (token, 512-channel group) rows on a wave takes eight tokens, below it four: the halo read
 // again is smaller, but fewer waves are in flight.  Measured in bf16, four against eight tokens: 18.9 / 19.6
 // us at 31,200 rows, 22.6 / 23.1 at 40,950, 29.9 / 28.9 at 65,520, 43.6 / 41.6 at 81,900, 159 / 146 at
-// 327,600; two tokens gain at most 0.4 us on the smallest inputs and lose from 10,000 rows on.
+// 327,600; in fp32 76.1 / 73.5 at 81,900, 82 / 74 at 200,000, 277 / 264 at 327,600.  Two tokens gain at most
+// 0.4 us on the smallest inputs and lose from 10,000 rows on.
 constexpr int64_t kConvRows8 = 49152;
 
 __device__ __forceinline__ float sigmoid_f(float z) {
@@ -78,10 +81,10 @@ __device__ __forceinline__ void seq_of(int64_t t, const ConvArgs& a, int& n, int
 template <typename TX, int W, int HL, int R>
 __global__ __launch_bounds__(WAVE * kConvWaves) void conv1d_rows_kernel(ConvArgs a, int64_t n_runs, int fold_state) {
   // the workgroup's waves take consecutive runs of one channel group, which share their halo rows
-  const int ncg = (a.D + 511) / 512;
-  const int64_t run = (int64_t)(blockIdx.x / ncg) * kConvWaves + threadIdx.x / WAVE;
+  const unsigned ncg = (a.D + 511) / 512, block = blockIdx.y * gridDim.x + blockIdx.x;
+  const int64_t run = (int64_t)(block / ncg) * kConvWaves + threadIdx.x / WAVE;
   if (run >= n_runs) return;
-  const int c0 = (int)(blockIdx.x % ncg) * 512 + 8 * lane_id();
+  const int c0 = (int)(block % ncg) * 512 + 8 * lane_id();
   const bool ok = c0 < a.D;
   const int cc = ok ? c0 : 0;                        // lanes past D load channel 0 and store nothing
   const int64_t t_begin = run * R;
@@ -225,11 +228,13 @@ template <typename TX, int W, int R>
 int launch_conv_rows(const ConvArgs& a, bool fold, hipStream_t s) {
   const int64_t n_runs = (a.total_tokens + R - 1) / R;
   const int64_t blocks = (n_runs + kConvWaves - 1) / kConvWaves * ((a.D + 511) / 512);
+  // a row of the grid holds fewer than 2^32 threads, which 2^29 tokens of 8 channels exceed
+  const int64_t row = std::min<int64_t>(blocks, 1 << 22), rows = (blocks + row - 1) / row;
   switch (a.head_lanes) {
 #define KGDN_CONV_CASE(HL)                                                                                     \
     case HL:                                                                                                   \
-      hipLaunchKernelGGL((conv1d_rows_kernel<TX, W, HL, R>), dim3((unsigned)blocks), dim3(WAVE * kConvWaves),  \
-                         0, s, a, n_runs, (int)fold);                                                          \
+      hipLaunchKernelGGL((conv1d_rows_kernel<TX, W, HL, R>), dim3((unsigned)row, (unsigned)rows),               \
+                         dim3(WAVE * kConvWaves), 0, s, a, n_runs, (int)fold);                                 \
       break;
     KGDN_CONV_CASE(0) KGDN_CONV_CASE(8) KGDN_CONV_CASE(16) KGDN_CONV_CASE(32) KGDN_CONV_CASE(64)
 #undef KGDN_CONV_CASE

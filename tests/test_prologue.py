@@ -168,6 +168,22 @@ def test_gpu_conv_run_edges(cid, B, T, D, W, cu, dt):
 
 
 @pytest.mark.gpu
+def test_gpu_conv_more_tokens_than_one_grid_row():
+    """8 channels and 2^29 + 40 tokens: 2^24 + 2 workgroups of 256 threads, past the 2^32 threads of a grid's row."""
+    import kairos_gdn
+    T, D = 2 ** 29 + 40, 8
+    gen = torch.Generator(device="cuda").manual_seed(0)
+    part = torch.randn(2 ** 16 + 3, D, device="cuda", generator=gen).to(torch.bfloat16)
+    x = part.repeat(-(-T // part.shape[0]), 1)[:T].contiguous()[None]
+    w = torch.randn(D, 4, device="cuda", generator=gen)
+    y, ht = kairos_gdn.causal_conv1d(x, w, activation="silu", output_final_state=True)
+    assert torch.equal(ht[0], x[0, -4:].T)
+    for t in (3, 2 ** 20, 2 ** 28 + 5, 2 ** 29 - 100, T - 64):
+        want, _ = kairos_gdn.causal_conv1d(x[:, t - 3:t + 64].contiguous(), w, activation="silu")
+        assert torch.equal(y[:, t:t + 64], want[:, 3:]), t
+
+
+@pytest.mark.gpu
 def test_gpu_short_convolution_module_prefill_then_decode():
     import kairos_gdn
     if not torch.cuda.is_available():
