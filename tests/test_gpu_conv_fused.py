@@ -81,8 +81,10 @@ CASES = [
 
 
 @pytest.mark.parametrize("name,shape,cu,cache,bias,wdt,l2", CASES, ids=[c[0] for c in CASES])
-def test_fused_conv_against_oracle(name, shape, cu, cache, bias, wdt, l2):
+def test_fused_conv_against_oracle(name, shape, cu, cache, bias, wdt, l2, monkeypatch):
     B, T, H, K, V = shape
+    if "pipelined" in name:
+        monkeypatch.setenv("KAIROS_GDN_WIDE_PIPE", "4")
     note(f"fused prologue {name}: B={B} T={T} H={H} K={K} V={V} cu={cu} cache={cache} bias={bias} {wdt} l2={l2}")
     x = make_case(B, T, H, K, V, seed=T + K + V, cu=cu, cache=cache, bias=bias, wdt=wdt, l2=l2)
     o, ht, caches = run_fused(x, l2, wdt)
@@ -98,14 +100,21 @@ def test_fused_conv_against_oracle(name, shape, cu, cache, bias, wdt, l2):
         np.testing.assert_array_equal(caches[i].float().cpu().numpy(), c_ref[n])
 
 
-@pytest.mark.parametrize("shape,cu", [((1, 700, 2, 256, 512), None), ((1, 400, 2, 256, 256), [0, 1, 4, 130, 400])])
-def test_fused_conv_equals_two_step_bit_for_bit(shape, cu):
-    """Without the L2 norm the fused call gives the bits of causal_conv1d on each projection followed by
-    chunk_gated_delta_rule (both through this library's kernels)."""
+@pytest.mark.parametrize("shape,cu,pipe", [((1, 700, 2, 256, 512), None, None), ((1, 700, 2, 256, 512), None, ("4", "1.4")),
+                                           ((2, 700, 2, 256, 512), None, ("2", "3")),
+                                           ((1, 400, 2, 256, 256), [0, 1, 4, 130, 400], None)])
+def test_fused_conv_equals_two_step_bit_for_bit(shape, cu, pipe, monkeypatch):
+    """Without the L2 norm the fused call, in one part and in parts (whose first rows take their halo from the
+    part before), gives the bits of causal_conv1d on each projection followed by chunk_gated_delta_rule in one
+    part (both through this library's kernels)."""
     B, T, H, K, V = shape
-    note(f"fused prologue vs two-step HIP path: {shape} cu={cu}")
+    note(f"fused prologue vs two-step HIP path: {shape} cu={cu} pipe={pipe}")
     x = make_case(B, T, H, K, V, seed=7 + T, cu=cu, cache=True, bias=True, l2=False)
+    if pipe:
+        monkeypatch.setenv("KAIROS_GDN_WIDE_PIPE", pipe[0])
+        monkeypatch.setenv("KAIROS_GDN_WIDE_PIPE_GROWTH", pipe[1])
     o, ht, caches = run_fused(x, False)
+    monkeypatch.setenv("KAIROS_GDN_WIDE_PIPE", "1")
     d = lambda a, dt=torch.bfloat16: None if a is None else torch.from_numpy(np.ascontiguousarray(a)).to("cuda", dt)  # noqa: E731
     cu_t = torch.tensor(cu, dtype=torch.int64, device="cuda") if cu else None
     ys = []

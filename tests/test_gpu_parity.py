@@ -345,6 +345,21 @@ def test_model_head_dims_pipeline_parts(with_h0, monkeypatch):
         assert torch.equal(ht, ht1), (parts, growth)
 
 
+@pytest.mark.parametrize("mark", ["0", "1", "2"])
+def test_model_head_dims_pipeline_marks(mark, monkeypatch):
+    """Whatever releases the next part's prepare (a marker kernel before the recurrence part, one on a stream of
+    its own, an event), two sequences in 4 parts give the bits of one part, call after call on one workspace."""
+    note(f"K=256 pipeline mark={mark}")
+    x = make_inputs(2, 64 * 12 + 37, 2, 256, 128, seed=44, dtype="bf16")
+    monkeypatch.setenv("KAIROS_GDN_WIDE_PIPE", "1")
+    o1, ht1 = run_gpu(x, "bf16")
+    monkeypatch.setenv("KAIROS_GDN_WIDE_PIPE", "4")
+    monkeypatch.setenv("KAIROS_GDN_WIDE_PIPE_MARK", mark)
+    for _ in range(3):
+        o, ht = run_gpu(x, "bf16")
+        assert torch.equal(o, o1) and torch.equal(ht, ht1)
+
+
 @pytest.mark.parametrize("H,V,nt", [(5, 512, 257), (10, 64, 210), (20, 512, 155), (20, 512, 410)],
                          ids=["2x3", "4x1.4_narrow", "2x1.4", "4x1.4"])
 def test_model_head_dims_default_parts(H, V, nt, monkeypatch):

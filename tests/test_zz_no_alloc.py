@@ -60,7 +60,8 @@ def _run(d, noalloc):
 
 
 @pytest.mark.gpu
-def test_noalloc_matches_chunk_fwd_on_two_calls():
+def test_noalloc_matches_chunk_fwd_on_two_calls(monkeypatch):
+    monkeypatch.setenv("KAIROS_GDN_WIDE_PIPE", "4")      # chunk_fwd in parts at K = 256, noalloc always in one
     cases = [
         ("B=2 T=3000 H=4 K=V=128 (several segments per sequence)", _problem(2, 3000, 4, 128, 128, seed=71)),
         ("varlen T=700 H=2 K=V=64, cu=[0, 1, 300, 700] (smaller)",
@@ -92,3 +93,44 @@ def test_noalloc_refuses_problems_beyond_the_static_array():
                                           _lib.BF16, _lib.BF16, _lib.F32, _lib.BF16, _lib.F32, K ** -0.5, 1, None)
     assert rc == _lib.EWORKSPACE
     assert b"static" in lib.kairos_gdn_last_error()
+
+
+def test_noalloc_refuses_packed_batches_beyond_the_static_array():
+    """Four packed sequences that fit the array with neither plan of segments."""
+    lib = _lib.load()
+    x, H, K = 16, 20, 128
+    rc = lib.kairos_gdn_chunk_fwd_noalloc(x, x, x, x, x, None, None, None, x, None, x, 4, 1, 90000, H, K, K, _lib.BF16,
+                                          _lib.BF16, _lib.F32, _lib.BF16, _lib.F32, K ** -0.5, 0, None)
+    assert rc == _lib.EWORKSPACE
+    assert b"static" in lib.kairos_gdn_last_error()
+
+
+@pytest.mark.gpu
+def test_noalloc_packed_batch_that_fits_with_fewer_segments(monkeypatch):
+    """A packed batch whose workspace exceeds the array runs with the longer segments that fit: the bits of
+    chunk_fwd cut that way."""
+    monkeypatch.delenv("KAIROS_GDN_SEG_CHUNKS", raising=False)
+    lib = _lib.load()
+    H, K = 20, 128
+    cu = [0, 3000, 21000, 26500, 66000]
+    T, N = cu[-1], len(cu) - 1
+    cap = lib.kairos_gdn_chunk_fwd_noalloc_max_bytes()
+    assert lib.kairos_gdn_chunk_fwd_workspace_size(1, T, H, K, K, N, _lib.BF16, _lib.BF16, 0) > cap
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    bound = T // 64 + N                                  # all segments of the longer plan fit the CUs at once
+    longer = -(-bound * H // max(cus - N * H, cus // 2))
+    assert longer > lib.kairos_gdn_segment_chunks(1, T, H, N)
+    print(f"noalloc packed batch T={T} H={H} K=V={K}, segments of {longer}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    r = lambda *sh: torch.randn(*sh, device="cuda", generator=gen)  # noqa: E731
+    unit = lambda t: (t / t.norm(dim=-1, keepdim=True)).to(torch.bfloat16)  # noqa: E731
+    d = dict(q=unit(r(1, T, H, K)), k=unit(r(1, T, H, K)), v=r(1, T, H, K).to(torch.bfloat16), g=-0.02 * r(1, T, H).abs(),
+             beta=torch.sigmoid(r(1, T, H)).to(torch.bfloat16), h0=0.02 * r(N, H, K, K),
+             cu=torch.tensor(cu, device="cuda"), shape=(1, T, H, K, K, N), dt=_lib.BF16, l2=0)
+    o, ht = _run(d, noalloc=True)
+    short, _ = _run(d, noalloc=False)
+    monkeypatch.setenv("KAIROS_GDN_SEG_CHUNKS", str(longer))
+    want, ht_want = _run(d, noalloc=False)
+    assert torch.isfinite(o.float()).all() and torch.isfinite(ht).all()
+    assert torch.equal(o, want) and torch.equal(ht, ht_want)
+    assert not torch.equal(o, short)                     # the packed plan's segments give other roundings
