@@ -34,7 +34,8 @@ constexpr int kConvWaves = 4;
 // again is smaller, but fewer waves are in flight.  Measured in bf16, four against eight tokens: 18.9 / 19.6
 // us at 31,200 rows, 22.6 / 23.1 at 40,950, 29.9 / 28.9 at 65,520, 43.6 / 41.6 at 81,900, 159 / 146 at
 // 327,600; in fp32 76.1 / 73.5 at 81,900, 82 / 74 at 200,000, 277 / 264 at 327,600.  Two tokens gain at most
-// 0.4 us on the smallest inputs and lose from 10,000 rows on.
+// 0.4 us on the smallest inputs and lose from 10,000 rows on.  In bf16 with the L2 norm four everywhere: eight
+// need 181 VGPRs, two waves a SIMD (181 / 163 us at 327,600 rows, 49 / 43 at 81,900).
 constexpr int64_t kConvRows8 = 49152;
 
 __device__ __forceinline__ float sigmoid_f(float z) {
@@ -77,7 +78,8 @@ __device__ __forceinline__ void seq_of(int64_t t, const ConvArgs& a, int& n, int
 // one wave on small ones, so a wave sends all its R + W - 1 row loads at once: walking a run of 64 rows
 // with the window in registers, each row waited for in turn, took 52 us at T = 1560, D = 5120 (now 12.5)
 // and 304 us at T = 32760, D = 10240 (now 277 us = 4.8 TB/s; a plain copy reaches 5.1).  The halo rows are
-// read again by the next wave, the workgroup's next, from the caches.
+// read again by the next wave, the workgroup's next, from the caches.  With the L2 norm the tokens' sums are
+// reduced together: at T = 32760, D = 5120 in bf16 224 us one after another, 163 so (166 the 64-row walk).
 template <typename TX, int W, int HL, int R>
 __global__ __launch_bounds__(WAVE * kConvWaves) void conv1d_rows_kernel(ConvArgs a, int64_t n_runs, int fold_state) {
   // the workgroup's waves take consecutive runs of one channel group, which share their halo rows
@@ -127,6 +129,8 @@ __global__ __launch_bounds__(WAVE * kConvWaves) void conv1d_rows_kernel(ConvArgs
     }
   };
   if (t_begin - P < bos) load_cache();
+  Vec8<TX> o[R];
+  float ss[R] = {};
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int64_t t = t_begin + r;
@@ -148,34 +152,37 @@ __global__ __launch_bounds__(WAVE * kConvWaves) void conv1d_rows_kernel(ConvArgs
 #pragma unroll
           for (int e = 0; e < 8; ++e) in[i][e] = hc[e * W + d + 1 + i];
       }
-    float out[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       float acc = bias[e];
 #pragma unroll
       for (int i = 0; i < W; ++i) acc = fmaf(wt[i][e], in[i][e], acc);
       if (a.silu) acc = acc * sigmoid_f(acc);
-      out[e] = round_to<TX>(acc);
-    }
-    if constexpr (HL > 0) {                          // per-head L2 norm over HL lanes of 8 channels
-      float ss = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) ss = fmaf(out[e], out[e], ss);
-#pragma unroll
-      for (int off = HL / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off, HL);
-      const float r1 = 1.0f / __builtin_sqrtf(ss + 1e-6f);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) out[e] *= r1;
+      acc = round_to<TX>(acc);
+      vset<TX>(o[r], e, acc);
+      if constexpr (HL > 0) ss[r] = fmaf(acc, acc, ss[r]);
     }
     if (!ok) continue;
-    Vec8<TX> o;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) vset<TX>(o, e, out[e]);
-    st8<TX>(y + t * a.D + c0, o);
+    if constexpr (HL == 0) st8<TX>(y + t * a.D + c0, o[r]);
     if (fold_state && t == eos - 1) {                // the final cache: the last token's own window
       TX* ht = static_cast<TX*>(a.ht) + ((int64_t)n * a.D + c0) * W;
 #pragma unroll
       for (int f = 0; f < 8 * W; ++f) ht[f] = from_f32<TX>(in[f % W][f / W]);
+    }
+  }
+  if constexpr (HL > 0) {                            // per-head L2 norm over HL lanes of 8 channels
+#pragma unroll
+    for (int off = HL / 2; off > 0; off >>= 1)
+#pragma unroll
+      for (int r = 0; r < R; ++r) ss[r] += __shfl_xor(ss[r], off, HL);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int64_t t = t_begin + r;
+      const float r1 = 1.0f / __builtin_sqrtf(ss[r] + 1e-6f);
+      if (t >= t_stop || !ok) break;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) vset<TX>(o[r], e, vget<TX>(o[r], e) * r1);
+      st8<TX>(y + t * a.D + c0, o[r]);
     }
   }
 }
@@ -224,23 +231,30 @@ __global__ __launch_bounds__(256) void to_f32_kernel(const void* src, int dt, fl
   if (i < n) dst[i] = ld_scalar(src, i, dt);
 }
 
-template <typename TX, int W, int R>
+template <typename TX, int W, int HL, int R>
 int launch_conv_rows(const ConvArgs& a, bool fold, hipStream_t s) {
   const int64_t n_runs = (a.total_tokens + R - 1) / R;
   const int64_t blocks = (n_runs + kConvWaves - 1) / kConvWaves * ((a.D + 511) / 512);
   // a row of the grid holds fewer than 2^32 threads, which 2^29 tokens of 8 channels exceed
   const int64_t row = std::min<int64_t>(blocks, 1 << 22), rows = (blocks + row - 1) / row;
+  hipLaunchKernelGGL((conv1d_rows_kernel<TX, W, HL, R>), dim3((unsigned)row, (unsigned)rows), dim3(WAVE * kConvWaves),
+                     0, s, a, n_runs, (int)fold);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+template <typename TX, int W>
+int launch_conv_w(const ConvArgs& a, bool fold, hipStream_t s) {
+  const bool r8 = a.total_tokens * ((a.D + 511) / 512) >= kConvRows8;
   switch (a.head_lanes) {
-#define KGDN_CONV_CASE(HL)                                                                                     \
-    case HL:                                                                                                   \
-      hipLaunchKernelGGL((conv1d_rows_kernel<TX, W, HL, R>), dim3((unsigned)row, (unsigned)rows),               \
-                         dim3(WAVE * kConvWaves), 0, s, a, n_runs, (int)fold);                                 \
-      break;
+#define KGDN_CONV_CASE(HL)                                                  \
+    case HL:                                                                \
+      if constexpr (W == 4 && (HL == 0 || sizeof(TX) == 4))                 \
+        if (r8) return launch_conv_rows<TX, W, HL, 8>(a, fold, s);          \
+      return launch_conv_rows<TX, W, HL, 4>(a, fold, s);
     KGDN_CONV_CASE(0) KGDN_CONV_CASE(8) KGDN_CONV_CASE(16) KGDN_CONV_CASE(32) KGDN_CONV_CASE(64)
 #undef KGDN_CONV_CASE
     default: return -2;
   }
-  return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 template <typename TX>
@@ -249,13 +263,12 @@ int launch_conv_t(const ConvArgs& a, hipStream_t s) {
   // hold empty sequences, which no wave visits
   const bool fold = a.ht != nullptr && a.cu == nullptr && a.total_tokens > 0;
   if (a.total_tokens > 0) {
-    const bool r8 = a.total_tokens * ((a.D + 511) / 512) >= kConvRows8;
     int rc = -2;
     switch (a.W) {
-      case 1: rc = launch_conv_rows<TX, 1, 4>(a, fold, s); break;
-      case 2: rc = launch_conv_rows<TX, 2, 4>(a, fold, s); break;
-      case 3: rc = launch_conv_rows<TX, 3, 4>(a, fold, s); break;
-      case 4: rc = r8 ? launch_conv_rows<TX, 4, 8>(a, fold, s) : launch_conv_rows<TX, 4, 4>(a, fold, s); break;
+      case 1: rc = launch_conv_w<TX, 1>(a, fold, s); break;
+      case 2: rc = launch_conv_w<TX, 2>(a, fold, s); break;
+      case 3: rc = launch_conv_w<TX, 3>(a, fold, s); break;
+      case 4: rc = launch_conv_w<TX, 4>(a, fold, s); break;
       default: return -2;
     }
     if (rc || fold) return rc;

@@ -167,6 +167,16 @@ def test_gpu_conv_run_edges(cid, B, T, D, W, cu, dt):
     test_gpu_causal_conv1d(cid, B, T, D, W, cu, True, dt, 0)
 
 
+# The norm over a run: short last runs, sequences ending inside one, every head dim, runs of 8 (fp32)
+@pytest.mark.gpu
+@pytest.mark.parametrize("hd", [64, 128, 256, 512])
+@pytest.mark.parametrize("B,T,D,cu,dt", [(3, 5, 512, None, "bf16"), (1, 21, 1536, [0, 1, 1, 4, 8, 9, 21], "bf16"),
+                                         (3, 820, 10240, None, "bf16"), (1, 2461, 10240, [0, 2, 1207, 2461], "fp32")],
+                         ids=["batch", "varlen", "long", "fp32_runs8"])
+def test_gpu_conv_run_norm(hd, B, T, D, cu, dt):
+    test_gpu_causal_conv1d(f"norm{hd}", B, T, D, 4, cu, True, dt, hd)
+
+
 @pytest.mark.gpu
 def test_gpu_conv_more_tokens_than_one_grid_row():
     """8 channels and 2^29 + 40 tokens: 2^24 + 2 workgroups of 256 threads, past the 2^32 threads of a grid's row."""
