@@ -802,7 +802,7 @@ def bench_prologue(args, dev):
         "config": {"workload": "kairos_gdn_causal_conv1d_fwd x3 (q, k: D=5120 with per-head L2 norm; v: D=10240), "
                                "bf16, W=4, caches out, + kairos_gdn_gates_fwd (T x 20)"},
         **timer.fields(res),
-        "roofline": {"bound": "hbm", "kernel": "conv1d_kernel", "achieved": gbs, "peak": PEAK_HBM_GBS,
+        "roofline": {"bound": "hbm", "kernel": "conv1d_rows_kernel", "achieved": gbs, "peak": PEAK_HBM_GBS,
                      "unit": "GB/s", "frac": gbs / PEAK_HBM_GBS, "alg_bytes": nbytes, "traffic": None},
     }), flush=True)
 
