@@ -31,15 +31,17 @@
  *    memory comes from the caller's `workspace`.  Entry points are reentrant;
  *    concurrent calls must use distinct workspaces.  One exception in how the
  *    work is queued: the fixed-length K = 256 forward of kairos_gdn_chunk_fwd
- *    (and of the _gated_norm / _conv calls) runs in parts on library streams
- *    of the current device (two, three with the gated norm, which runs by
- *    parts beside the last recurrence part), shared by every caller in the process
- *    (created on first use, default priority, kept until exit, enqueued under
- *    one process-wide lock), joined to `stream` by events: work queued on
- *    `stream` after the call sees its results, but such calls issued from
- *    different caller streams run one after another on the library streams.
- *    Under graph capture, for varlen batches, in kairos_gdn_chunk_fwd_noalloc
- *    and with KAIROS_GDN_WIDE_PIPE=1 everything runs on `stream`.
+ *    (and of the _gated_norm / _conv calls) runs long calls in two or four parts
+ *    (planned from the chunk and head count and the CUs the recurrence leaves):
+ *    the recurrence on `stream`, the later parts' prepares on a library stream of
+ *    the current device and the gated norm by parts on another, shared by every
+ *    caller in the process (created on first use, default priority, kept until
+ *    exit, enqueued under one process-wide lock) and ordered by events: work
+ *    queued on `stream` after the call sees its results.  Recurrences of calls
+ *    from different caller streams may overlap; their prepares (and norms) run
+ *    one after another.  Short calls run on `stream` alone, and so does everything
+ *    under graph capture, for varlen batches, in kairos_gdn_chunk_fwd_noalloc
+ *    and with KAIROS_GDN_WIDE_PIPE=1.
  *  - Return value: KAIROS_GDN_OK or an error code; kairos_gdn_last_error()
  *    returns the message of the calling thread's last failure.  No exception
  *    crosses the ABI.
@@ -145,7 +147,8 @@ size_t kairos_gdn_chunk_fwd_gated_norm_workspace_size(int64_t B, int64_t T, int6
  * fewer, longer segments, run with those).  Every call on one GPU shares that GPU's array:
  * calls that overlap on one GPU (concurrent streams or threads) race and must
  * be serialised by the caller.  Same results as kairos_gdn_chunk_fwd (same
- * kernels and, but for those batches, the same segments); calls made through it are not recorded by the timing hook. */
+ * kernels and, but for those batches, the same segments); calls made through it
+ * are not recorded by the timing hook. */
 int kairos_gdn_chunk_fwd_noalloc(const void* q, const void* k, const void* v, const void* g, const void* beta,
                                  const float* q_scale, const float* k_scale, const void* initial_state, void* o,
                                  float* final_state, const int64_t* cu_seqlens, int64_t n_seqs, int64_t B,

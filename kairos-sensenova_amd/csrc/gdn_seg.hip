@@ -242,7 +242,8 @@ __device__ __forceinline__ SegLoc locate_seg(int s, const SegGeom& G) {
 // (lane r % 16 + 16 (c % 32 / 8), element c % 8), so that seg_combine loads an operand as 1 KB in a row.
 // (From row-major maps each load took 64 bytes of 16 rows, twice the lines for the address unit, which
 // bounds its step: the combine of 512 chunks with 20 heads 29 -> 16 us, of a 60-chunk sequence beside five
-// short ones 25 -> 13.5.)  Linear over multiples of 16 rows or 32 columns and over rows below 16.
+// short ones 25 -> 13.5; seg_trans, whose lanes store 2 bytes each into 16 of a line, takes 2 to 4 us more.)
+// Linear over multiples of 16 rows or 32 columns and over rows below 16.
 template <int K>
 __device__ __forceinline__ constexpr int map_off(int r, int c) {
   return ((r >> 4) * (K / 32) + (c >> 5)) * 512 + 128 * ((c >> 3) & 3) + 8 * (r & 15) + (c & 7);
