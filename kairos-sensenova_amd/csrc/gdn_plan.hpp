@@ -27,14 +27,17 @@ struct PipePlan {
 // read ahead of the steps, and four parts by 1.4 keep more of it in the last cache (V = 64, 5 heads, 512
 // chunks: one part 1699, two by 3 1657, four 1459; 10 heads, 256 chunks 980 / 938 / 833; V = 128, 20 heads,
 // 128 chunks 538 / 494 / 474; with 1280 items one part is best, 20 heads of 64 chunks 196 / 210 / 229).
-constexpr PipePlan wide_pipe_plan(int64_t nt, int64_t seq_heads, int64_t vtiles, int64_t cus) {
+// `norm`: the gated norm runs by parts too, the last part's after everything else, so a smaller last part pays
+// earlier (20 heads, with the norm: 188 chunks 748 in two parts, 743 in four; 256 989 / 963; 375 1436 / 1381; two
+// sequences of 128 979 / 993).
+constexpr PipePlan wide_pipe_plan(int64_t nt, int64_t seq_heads, int64_t vtiles, int64_t cus, bool norm) {
   const int64_t items = nt * seq_heads, units = seq_heads * vtiles, slots = (units + cus - 1) / cus * cus;
   if (units <= cus ? 4 * (cus - units) < cus : 10 * (slots - units) < 3 * slots) return {1, 1.0};
   if (2 * units <= cus) {
     if (vtiles <= 2 && items >= 2048) return {4, 1.4};
     return {items >= 1280 && nt >= 128 ? 2 : 1, 3.0};
   }
-  return {items >= 8192 ? 4 : items >= 3072 ? 2 : 1, 1.4};
+  return {items >= (norm && units <= cus ? 4096 : 8192) ? 4 : items >= 3072 ? 2 : 1, 1.4};
 }
 
 }  // namespace kgdn

@@ -10,7 +10,7 @@ MAIN = r"""
 #include <cstdlib>
 #include "%s"
 int main(int, char** v) {
-  const kgdn::PipePlan p = kgdn::wide_pipe_plan(atoi(v[1]), atoi(v[2]), atoi(v[3]), 256);
+  const kgdn::PipePlan p = kgdn::wide_pipe_plan(atoi(v[1]), atoi(v[2]), atoi(v[3]), 256, atoi(v[4]) != 0);
   printf("%%d %%.1f", p.parts, p.growth);
 }
 """
@@ -36,4 +36,11 @@ def plan(tmp_path_factory):
     (512, 5, 1, "4 1.4"), (256, 10, 1, "4 1.4"), (128, 20, 2, "4 1.4"), (64, 20, 1, "1 3.0"), (32, 40, 2, "1 3.0"),
 ])
 def test_fastest_measured_form(plan, nt, heads, tiles, want):
-    assert plan(nt, heads, tiles) == want
+    assert plan(nt, heads, tiles, 0) == want
+
+
+@pytest.mark.parametrize("nt,heads,tiles,want", [(128, 20, 8, "1 1.4"), (256, 20, 8, "4 1.4"), (375, 20, 8, "4 1.4"),
+                                                 (512, 20, 8, "4 1.4"), (128, 40, 8, "2 1.4"), (512, 10, 8, "2 3.0"),
+                                                 (256, 20, 4, "2 3.0"), (256, 32, 8, "1 1.0")])
+def test_fastest_measured_form_with_the_norm_by_parts(plan, nt, heads, tiles, want):
+    assert plan(nt, heads, tiles, 1) == want
