@@ -372,8 +372,8 @@ size_t bwd_ws(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t n_s
 constexpr int kMaxParts = 16;
 
 // KAIROS_GDN_WIDE_PIPE sets the number of parts, KAIROS_GDN_WIDE_PIPE_GROWTH their growth.
-kgdn::PipePlan wide_pipe(int64_t nt, int64_t seq_heads, int64_t vtiles, bool norm) {
-  kgdn::PipePlan p = kgdn::wide_pipe_plan(nt, seq_heads, vtiles, kgdn::device_cus(), norm);
+kgdn::PipePlan wide_pipe(int64_t nt, int64_t seq_heads, int64_t vtiles, bool norm, bool conv) {
+  kgdn::PipePlan p = kgdn::wide_pipe_plan(nt, seq_heads, vtiles, kgdn::device_cus(), norm, conv);
   if (const char* e = std::getenv("KAIROS_GDN_WIDE_PIPE")) {
     const int n = std::atoi(e);
     p = {n < 1 ? 1 : n > kMaxParts ? kMaxParts : n, 1.4};
@@ -553,7 +553,7 @@ int run_staged(const Geometry& G, const void* q, const void* k, const void* v, c
     // the gated norm of part p's rows (per sequence: tokens [64 bnd[p], 64 bnd[p + 1]) of each)
     // on s5 once recurrence part p is done, beside the next part's recurrence
     const bool nparts = epi != nullptr && N <= 8 && norm_parts_on();
-    const kgdn::PipePlan plan = wide_pipe(nt, (int64_t)N * H, V / 64, nparts);
+    const kgdn::PipePlan plan = wide_pipe(nt, (int64_t)N * H, V / 64, nparts, conv3 != nullptr);
     const double growth = plan.growth;
     int P = plan.parts;
     if (nt < 2 * P) P = 1;

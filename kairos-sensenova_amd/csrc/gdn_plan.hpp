@@ -30,12 +30,17 @@ struct PipePlan {
 // `norm`: the gated norm runs by parts too, the last part's after everything else, so a smaller last part pays
 // earlier (20 heads, with the norm: 188 chunks 748 in two parts, 743 in four; 256 989 / 963; 375 1436 / 1381; two
 // sequences of 128 979 / 993).
-constexpr PipePlan wide_pipe_plan(int64_t nt, int64_t seq_heads, int64_t vtiles, int64_t cus, bool norm) {
+// `conv`: prepare convolves too and takes half as long again, so that with more than 10 heads it no longer ends
+// within a recurrence part a third of its length (16 heads, 375 chunks 1389 in two parts by 3, 1326 by 1.4, 1294 in
+// four; 188 chunks 754 / 703 / 729; V = 256, 20 heads, 375 chunks 1514 / 1462 / 1396; 10 heads 1209 / 1248 / 1223).
+constexpr PipePlan wide_pipe_plan(int64_t nt, int64_t seq_heads, int64_t vtiles, int64_t cus, bool norm, bool conv) {
   const int64_t items = nt * seq_heads, units = seq_heads * vtiles, slots = (units + cus - 1) / cus * cus;
   if (units <= cus ? 4 * (cus - units) < cus : 10 * (slots - units) < 3 * slots) return {1, 1.0};
   if (2 * units <= cus) {
     if (vtiles <= 2 && items >= 2048) return {4, 1.4};
-    return {items >= 1280 && nt >= 128 ? 2 : 1, 3.0};
+    const int two = items >= 1280 && nt >= 128 ? 2 : 1;
+    if (conv && seq_heads > 10) return {items >= 3584 ? 4 : two, 1.4};
+    return {two, 3.0};
   }
   return {items >= (norm && units <= cus ? 4096 : 8192) ? 4 : items >= 3072 ? 2 : 1, 1.4};
 }

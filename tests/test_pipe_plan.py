@@ -10,7 +10,7 @@ MAIN = r"""
 #include <cstdlib>
 #include "%s"
 int main(int, char** v) {
-  const kgdn::PipePlan p = kgdn::wide_pipe_plan(atoi(v[1]), atoi(v[2]), atoi(v[3]), 256, atoi(v[4]) != 0);
+  const kgdn::PipePlan p = kgdn::wide_pipe_plan(atoi(v[1]), atoi(v[2]), atoi(v[3]), 256, atoi(v[4]) & 1, atoi(v[4]) & 2);
   printf("%%d %%.1f", p.parts, p.growth);
 }
 """
@@ -44,3 +44,10 @@ def test_fastest_measured_form(plan, nt, heads, tiles, want):
                                                  (256, 20, 4, "2 3.0"), (256, 32, 8, "1 1.0")])
 def test_fastest_measured_form_with_the_norm_by_parts(plan, nt, heads, tiles, want):
     assert plan(nt, heads, tiles, 1) == want
+
+
+@pytest.mark.parametrize("nt,heads,tiles,want", [(188, 16, 8, "2 1.4"), (375, 16, 8, "4 1.4"), (188, 20, 4, "4 1.4"),
+                                                 (375, 12, 8, "4 1.4"), (375, 10, 8, "2 3.0"), (375, 20, 8, "2 1.4"),
+                                                 (94, 20, 8, "1 1.4"), (375, 5, 8, "2 3.0")])
+def test_fastest_measured_form_with_the_convolution(plan, nt, heads, tiles, want):
+    assert plan(nt, heads, tiles, 2) == want
