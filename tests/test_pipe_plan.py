@@ -33,7 +33,9 @@ def plan(tmp_path_factory):
     (256, 28, 8, "1 1.0"), (256, 32, 8, "1 1.0"), (512, 36, 8, "4 1.4"), (128, 40, 8, "2 1.4"), (512, 40, 8, "4 1.4"),
     (256, 48, 8, "1 1.0"), (128, 60, 8, "1 1.0"), (256, 64, 8, "1 1.0"), (128, 80, 8, "1 1.0"),
     (64, 5, 8, "1 3.0"), (512, 5, 8, "2 3.0"), (512, 10, 8, "2 3.0"), (64, 20, 4, "1 3.0"), (128, 20, 4, "2 3.0"),
-    (512, 5, 1, "4 1.4"), (256, 10, 1, "4 1.4"), (128, 20, 2, "4 1.4"), (64, 20, 1, "1 3.0"), (32, 40, 2, "1 3.0"),
+    (512, 5, 1, "4 1.4"), (256, 10, 1, "4 1.4"), (128, 20, 2, "4 1.4"), (64, 20, 1, "1 3.0"), (32, 40, 2, "1 1.4"),
+    (64, 40, 2, "2 1.4"), (64, 40, 1, "4 1.4"), (47, 64, 1, "2 1.4"),
+    (256, 16, 8, "2 1.4"), (512, 14, 8, "2 3.0"), (375, 20, 4, "2 3.0"), (256, 32, 4, "4 1.4"), (512, 32, 4, "4 1.4"),
 ])
 def test_fastest_measured_form(plan, nt, heads, tiles, want):
     assert plan(nt, heads, tiles, 0) == want
@@ -41,7 +43,8 @@ def test_fastest_measured_form(plan, nt, heads, tiles, want):
 
 @pytest.mark.parametrize("nt,heads,tiles,want", [(128, 20, 8, "1 1.4"), (256, 20, 8, "4 1.4"), (375, 20, 8, "4 1.4"),
                                                  (512, 20, 8, "4 1.4"), (128, 40, 8, "2 1.4"), (512, 10, 8, "2 3.0"),
-                                                 (256, 20, 4, "2 3.0"), (256, 32, 8, "1 1.0")])
+                                                 (256, 20, 4, "2 3.0"), (256, 32, 8, "1 1.0"),
+                                                 (512, 16, 8, "4 1.4"), (256, 32, 4, "4 1.4")])
 def test_fastest_measured_form_with_the_norm_by_parts(plan, nt, heads, tiles, want):
     assert plan(nt, heads, tiles, 1) == want
 
