@@ -777,7 +777,7 @@ __global__ __launch_bounds__(NT_F + FL * WAVE) void wide_fused_kernel(WideFusedA
       }
     }
     // rows past the chunk's end are copies of its first, and an infinite one times their zero gate would be NaN
-    // (here, where the products end, the check is free; in the update it cost 1.5% of the step)
+    // (here, where the products end, only the short chunk pays, 0.3 us; in the update every step paid 1.5%)
     if (nv < C) {
 #pragma unroll
       for (int tm = 0; tm < 4; ++tm)
