@@ -777,7 +777,8 @@ __global__ __launch_bounds__(NT_F + FL * WAVE) void wide_fused_kernel(WideFusedA
       }
     }
     // rows past the chunk's end are copies of its first, and an infinite one times their zero gate would be NaN
-    // (here, where the products end, only the short chunk pays, 0.3 us; in the update every step paid 1.5%)
+    // (clearing them here, where the products end, costs nothing measurable: V = 512, H = 5, T = 32760 1198 to
+    // 1199 us, against 1217 with the check in the update; H = 20, T = 1560 88 us before and after, within 0.5 us)
     if (nv < C) {
 #pragma unroll
       for (int tm = 0; tm < 4; ++tm)
